@@ -49,7 +49,7 @@ typedef struct s3d_options {
                               0 off, 1 FP32 compensation words,
                               2 BF16 compensation words                   */
     int device;            /* HIP device ordinal                          */
-    int xcd_remap;         /* 1: give each XCD a contiguous element range */
+    int xcd_remap;         /* 1: give each XCD contiguous runs of elements */
     int bf16_static;       /* FP32: store the moduli, tau and dt/M in BF16 */
     int state_buffers;     /* stress, compensation and memory variables:
                               2 (and 0, the default): two blocks, each step

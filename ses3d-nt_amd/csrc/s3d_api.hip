@@ -1043,11 +1043,8 @@ int batch_build_group_e(BatchGroup &G)
     // come from HBM once per tile and from cache for the other members.
     bool interleave = n > 1;
     for (int q = 1; q < n && interleave; ++q) interleave = model_of(G.sims[q]) == model_of(G.sims[0]);
-    // the element launch is padded to a multiple of 8 workgroups (idle ones
-    // own simulation -1) so its XCD-aware block order applies
-    auto owners = [n](const std::vector<int> &st, int pad8, bool inter) {
-        const int total = pad8 ? (st[n] + 7) / 8 * 8 : st[n];
-        std::vector<int2> o(total, make_int2(-1, 0));
+    auto owners = [n](const std::vector<int> &st, bool inter) {
+        std::vector<int2> o(st[n]);
         if (inter) {
             const int per = st[1] - st[0];   // members share the mesh and tile
             for (int w = 0; w < per; ++w)
@@ -1059,9 +1056,8 @@ int batch_build_group_e(BatchGroup &G)
         return o;
     };
     // receivers differ between members: their launch stays member-major
-    const std::vector<int2> eo = owners(es, 1, interleave), no = owners(ns, 0, interleave),
-                            ro = owners(rs, 0, false);
-    G.ewg = (int)eo.size();
+    const std::vector<int2> eo = owners(es, interleave), no = owners(ns, interleave),
+                            ro = owners(rs, false);
     HIPCHK(hipMalloc(&G.d_eargs, sizeof(ElemArgs<R>) * 2 * n));
     HIPCHK(hipMalloc(&G.d_nargs, sizeof(NodeArgs<R>) * n));
     HIPCHK(hipMalloc(&G.d_rargs, sizeof(RecArgs<R>) * 2 * n));

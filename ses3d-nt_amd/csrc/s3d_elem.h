@@ -24,13 +24,34 @@ struct Shape {
     static constexpr int NT = ((EPB * NP + 63) / 64) * 64;
 };
 
-__device__ inline int remap_block(int b, int G, int remap)
+// Workgroup order of the element kernel: dispatch deals consecutive workgroups
+// to the 8 XCDs in turn; with `on`, XCD x runs the tiles of chunks x, x + 8,
+// x + 16, ... of XCD_CHUNK consecutive tiles each. Neighbours along theta
+// (shared velocity and force nodes) still meet in one L2, and all XCDs work
+// in one window of memory (8 chunks) that moves through the state block. With
+// one contiguous range of tiles per XCD eight windows far apart compete for
+// the DRAM rows: element kernel at order 4, 96x96x48, FP32 with five memory
+// words, 2.43 ms with ranges, 2.28 ms with chunks; FP64 at 48x48x24 0.55 and
+// 0.52 ms. Chunks of 4 to 64 tiles are within 3 % of each other at orders 2
+// to 7, and 16 within 1 % of the best of each; alternating the tiles of two
+// planes inside the order (so that the upper tile finds the shared velocity
+// nodes in L2) costs 1 to 5 % and is not done. The workgroups past the last
+// whole group of 8 chunks keep the plain order.
+// A launch of at most XCD_RESIDENT workgroups is in flight as a whole, there
+// is no moving window, and what its XCD wrote in the last step may still be in
+// that L2: ranges (12x12x8, order 4, FP64: 12.8 us, 13.2 us with chunks; at
+// 2048 workgroups 25.5 and 26.2 us, at 4608 60.0 and 55.2 us).
+constexpr int XCD_CHUNK = 16;
+constexpr int XCD_RESIDENT = 2048;
+
+__device__ inline int chunk_block(int b, int G, int on)
 {
-    // Dispatch sends consecutive workgroups to consecutive XCDs (8 on MI355X).
-    // Remapping gives each XCD a contiguous range of elements, so element
-    // neighbours (shared velocity / force nodes) meet in the same L2.
-    if (!remap || (G & 7)) return b;
-    return (b & 7) * (G >> 3) + (b >> 3);
+    constexpr int group = 8 * XCD_CHUNK;
+    if (!on) return b;
+    if (G <= XCD_RESIDENT) return (G & 7) ? b : (b & 7) * (G >> 3) + (b >> 3);
+    if (b >= G / group * group) return b;
+    const int g = b / group, r = b - g * group;
+    return g * group + (r & 7) * XCD_CHUNK + (r >> 3);
 }
 
 template <int P>
@@ -640,31 +661,11 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R> &a, int blk)
     }
 }
 
-// Plane-pair tile order: launch position t runs the tile at position q of
-// plane 2m + s, s fastest, so the tile above follows the tile below and
-// finds the velocity blocks they share (its own, the lower tile's z+1 face)
-// still in L2; in plane order they came back from memory a plane of tiles
-// later. A permutation of the tiles (identity where a tile would straddle
-// two planes, and for the last plane of an odd count): the arithmetic is
-// unchanged. Fewer velocity re-reads from memory; the time gain at
-// 192x192x96 is within run-to-run noise (at most about 0.5 %).
-template <int EPB>
-__device__ inline int plane_pair_tile(int t, int nx, int ny, int nz)
-{
-    const int pe = nx * ny;
-    if (pe % EPB) return t;
-    const int TP = pe / EPB;   // tiles per plane
-    if (t >= (nz & ~1) * TP) return t;
-    const int m = t / (2 * TP), r = t - m * 2 * TP;
-    return (2 * m + (r & 1)) * TP + (r >> 1);
-}
-
 template <int P, int E, typename R, int VM, bool S16, int KS, int LL>
 __global__ void __launch_bounds__((Shape<P, E>::NT))
 elem_kernel(const ElemArgs<R> a)
 {
-    const int t = remap_block(blockIdx.x, gridDim.x, a.remap);
-    elem_body<P, E, R, VM, S16, KS, LL>(a, plane_pair_tile<Shape<P, E>::EPB>(t, a.nx, a.ny, a.nz));
+    elem_body<P, E, R, VM, S16, KS, LL>(a, chunk_block(blockIdx.x, gridDim.x, a.remap));
 }
 
 template <int P, int E, typename R, int VM, int KS, int LL>
@@ -672,11 +673,9 @@ __global__ void __launch_bounds__((Shape<P, E>::NT))
 elem_kernel_batch(const ElemArgs<R> *__restrict__ args, const int2 *__restrict__ own)
 {
     // (simulation, its workgroup index), in XCD-aware order over the whole
-    // batch: each XCD works through a contiguous range of simulations
-    const int2 o = own[remap_block(blockIdx.x, gridDim.x, 1)];
-    if (o.x < 0) return;   // padding workgroup
-    const ElemArgs<R> &a = args[o.x];
-    elem_body<P, E, R, VM, false, KS, LL>(a, plane_pair_tile<Shape<P, E>::EPB>(o.y, a.nx, a.ny, a.nz));
+    // batch
+    const int2 o = own[chunk_block(blockIdx.x, gridDim.x, 1)];
+    elem_body<P, E, R, VM, false, KS, LL>(args[o.x], o.y);
 }
 
 }  // namespace s3d

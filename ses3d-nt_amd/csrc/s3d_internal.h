@@ -101,7 +101,7 @@ struct Static16 {
 template <typename R>
 struct ElemArgs {
     int nx, ny, nz, nel;
-    int remap;                 // XCD-aware block order
+    int remap;                 // XCD-aware block order (chunk_block)
     gptr<const int> it_dev;    // iterations completed so far (device counter);
                                // this launch computes iteration *it_dev + 1
     int nt;

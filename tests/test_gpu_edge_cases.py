@@ -8,7 +8,7 @@ import pytest
 
 from helpers import random_model, rel_l2, small_grid
 from ses3d_amd import api
-from test_gpu_parity import FIELDS, _pair, _random_state
+from test_gpu_parity import FIELDS, PARAMS, _pair, _random_state
 
 pytestmark = pytest.mark.gpu
 
@@ -60,6 +60,34 @@ def test_plane_pair_order_matches_oracle(tile, nz):
         for f in FIELDS:
             assert rel_l2(s.get(f), o.get(f)) < tol, (precision, tile, f)
         s.close()
+
+
+@pytest.mark.parametrize("shape", [(8, 16, 16), (13, 15, 11), (17, 11, 11), (16, 16, 9), (13, 14, 13)])
+def test_workgroup_orders_match_oracle(shape):
+    """One element per workgroup, so the shapes are 2048 and 2145 workgroups
+    (8 x 256, and just past the resident limit), 2057 (a multiple of neither
+    8 nor 128), 2304 (whole groups of 8 chunks) and 2366 (a tail): every
+    element is advanced once in the XCD-aware order, as the oracle has it, and
+    bit for bit as in the plain order."""
+    nx, ny, nz = shape
+    grid = small_grid(nx=nx, ny=ny, nz=nz, lpd=2)
+    rng = np.random.default_rng(17)
+    model = random_model(grid, rng)
+    o, s = _pair(grid, model, precision="fp32")
+    plain = api.Simulation(grid, "fp32", xcd_remap=False)
+    for k, arr in model.items():
+        plain.set_model(PARAMS[k][1], arr)
+    plain.init()
+    _random_state(o, s, grid, rng)
+    for f in FIELDS:
+        plain.set(f, o.get(f))
+    for x in (s, plain):
+        x.set_tile(1)
+        x.step(3)
+    o.step(3)
+    for f in FIELDS:
+        assert rel_l2(s.get(f), o.get(f)) < 1e-5, (shape, f)
+        assert np.array_equal(s.get(f), plain.get(f)), (shape, f)
 
 
 def test_run_without_sources_or_receivers():
