@@ -9,12 +9,14 @@
 #include "s3d_launch.h"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <type_traits>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 using namespace s3d;
@@ -186,7 +188,7 @@ struct s3d_ctx {
     void *v[3] = {}, *lo[3] = {}, *dt_inv_mm = nullptr, *sig = nullptr, *sig_lo = nullptr,
          *mem = nullptr, *lam = nullptr, *mu = nullptr, *tau = nullptr, *rho = nullptr,
          *ca = nullptr, *cb = nullptr, *cc = nullptr, *force = nullptr, *tth = nullptr, *mat = nullptr,
-         *grad_rho = nullptr, *grad_stage = nullptr,   // FP64 density; 3 snapshot components
+         *grad_rho = nullptr,   // FP64 density [nel][NP]
          *dgrad = nullptr,   // FP64 displacement gradient [nel][6][NP], see s3d_enable_displacement_gradient
          *curl_parts = nullptr,   // FP64 [nel][6][NP], see s3d_capture_curl_strain
          *tr = nullptr, *wdev = nullptr;
@@ -734,16 +736,277 @@ struct CflRun {
     }
 };
 
-template <int P, typename R>
-struct ExpandRun {
-    static int run(s3d_ctx *c, const void *src, const void *lo, double *dst)
+// ---- fields to and from the host ----
+// A field crosses in chunks of at most IO_BYTES: export_field / import_field
+// work on a chunk in pinned host memory, and host threads copy between it and
+// the caller's array, each with a pinned buffer and an event of its own, so
+// that the copies of some chunks (and the first touch of the caller's pages)
+// run while the host link carries others: a velocity component at 96x96x48,
+// order 4 (442 MB into fresh pages) takes 45 ms on one thread, 16.8 ms on 4,
+// 13.4 ms on 8 and 16 threads (into touched pages 9.4 ms, 47 GB/s); chunks of
+// 2 MB 14.2 ms, 1 MB 16.5 ms. 32 MB: 1.29 ms on 4 threads, 1.48 ms on 8, so
+// the threads grow with the chunks. (One hipMemcpy from a device buffer:
+// 44 ms, and 254 ms for a stress component whose compensation the host
+// subtracted.) Buffers are taken from a process-wide list for the duration of
+// one call, at most IO_KEPT sets per device stay on it, and the last
+// simulation of a device frees them.
+constexpr int IO_THREADS = 8;
+constexpr size_t IO_BYTES = 4u << 20;
+constexpr size_t IO_KEPT = 2;
+
+struct IoBuffers {
+    int dev = 0;
+    char *buf[IO_THREADS] = {};
+    hipEvent_t ev[IO_THREADS] = {};
+};
+
+std::mutex g_io_mutex;
+std::vector<IoBuffers *> g_io_free;
+int g_live[MAX_DEVICES] = {};   // simulations per device
+
+void io_delete(IoBuffers *b)
+{
+    for (int t = 0; t < IO_THREADS; ++t) {
+        if (b->ev[t]) (void)hipEventDestroy(b->ev[t]);
+        if (b->buf[t]) (void)hipHostFree(b->buf[t]);
+    }
+    delete b;
+}
+
+IoBuffers *io_acquire(int dev)
+{
     {
-        hipLaunchKernelGGL((expand_unique<P, R>), dim3(nblocks(c->nn, 256)), dim3(256), 0, c->stream,
-                           (const R *)src, (const R *)(c->kv == 1 ? lo : nullptr),
-                           (const bf16 *)(c->kv == 2 ? lo : nullptr),
-                           dst, c->g.nx, c->g.ny, c->g.nz);
-        HIPCHK(hipGetLastError());
-        return 0;
+        std::lock_guard<std::mutex> lock(g_io_mutex);
+        for (size_t q = 0; q < g_io_free.size(); ++q)
+            if (g_io_free[q]->dev == dev) {
+                IoBuffers *b = g_io_free[q];
+                g_io_free.erase(g_io_free.begin() + q);
+                return b;
+            }
+    }
+    IoBuffers *b = new IoBuffers();
+    b->dev = dev;
+    return b;
+}
+
+void io_release(IoBuffers *b)
+{
+    {
+        std::lock_guard<std::mutex> lock(g_io_mutex);
+        size_t kept = 0;
+        for (const IoBuffers *f : g_io_free) kept += f->dev == b->dev;
+        if (kept < IO_KEPT && b->dev < MAX_DEVICES && g_live[b->dev] > 0) {
+            g_io_free.push_back(b);
+            return;
+        }
+    }
+    io_delete(b);
+}
+
+// a simulation of the device is created (+1) or destroyed (-1)
+void io_live(int dev, int d)
+{
+    std::vector<IoBuffers *> gone;
+    if (dev < 0 || dev >= MAX_DEVICES) return;
+    {
+        std::lock_guard<std::mutex> lock(g_io_mutex);
+        g_live[dev] += d;
+        if (g_live[dev] > 0) return;
+        for (size_t q = g_io_free.size(); q-- > 0;)
+            if (g_io_free[q]->dev == dev) {
+                gone.push_back(g_io_free[q]);
+                g_io_free.erase(g_io_free.begin() + q);
+            }
+    }
+    for (IoBuffers *b : gone) io_delete(b);
+}
+
+// thread t's buffer, allocated by its first use
+hipError_t io_buffer(IoBuffers *b, int t)
+{
+    if (!b->buf[t])
+        if (hipError_t e = hipHostMalloc((void **)&b->buf[t], IO_BYTES, hipHostMallocPortable)) return e;
+    if (!b->ev[t]) return hipEventCreateWithFlags(&b->ev[t], hipEventDisableTiming);
+    return hipSuccess;
+}
+
+// Chunks of `fields` fields of NP x nel values that share one buffer: whole
+// rows of elements where IO_N node rows of them fit, else pieces of rows.
+struct IoPlan {
+    long ne, ce;   // elements per chunk, chunks along the elements
+    int nn, cn;    // nodes per chunk, chunks along the nodes
+};
+
+IoPlan io_plan(const s3d_ctx *c, int fields)
+{
+    const long words = (long)(IO_BYTES / sizeof(double)) / fields;
+    IoPlan p;
+    if (c->nel * std::min(c->NP, IO_N) <= words) {
+        p.ne = c->nel;
+        p.nn = (int)std::min<long>(c->NP, words / c->nel);
+        if (p.nn < c->NP) p.nn = p.nn / IO_N * IO_N;
+    } else {
+        p.nn = std::min(c->NP, IO_N);
+        p.ne = words / p.nn / IO_E * IO_E;
+    }
+    p.ce = (c->nel + p.ne - 1) / p.ne;
+    p.cn = (c->NP + p.nn - 1) / p.nn;
+    return p;
+}
+
+// One chunk: its elements and nodes.
+struct IoChunk {
+    long e0;
+    int ne, n0, nn;
+    dim3 grid() const { return dim3((ne + IO_E - 1) / IO_E, (nn + IO_N - 1) / IO_N); }
+};
+
+// Run `one(chunk, buffer, event)` for every chunk on up to IO_THREADS host
+// threads.
+template <typename F>
+int io_chunks(s3d_ctx *c, int fields, F one)
+{
+    const IoPlan p = io_plan(c, fields);
+    const long total = p.ce * p.cn;
+    IoBuffers *b = io_acquire(c->dev);
+    std::atomic<long> next(0);
+    std::atomic<int> bad(hipSuccess);
+    auto work = [&](int t) {
+        hipError_t e = hipSetDevice(c->dev);
+        if (e == hipSuccess) e = io_buffer(b, t);
+        for (long q; e == hipSuccess && bad.load() == hipSuccess && (q = next.fetch_add(1)) < total;) {
+            // consecutive chunks lie side by side in the caller's rows
+            IoChunk k;
+            k.e0 = q % p.ce * p.ne;
+            k.ne = (int)std::min(p.ne, c->nel - k.e0);
+            k.n0 = (int)(q / p.ce) * p.nn;
+            k.nn = std::min(p.nn, c->NP - k.n0);
+            e = one(k, (double *)b->buf[t], b->ev[t]);
+        }
+        if (e != hipSuccess) bad.store(e);
+    };
+    const int want = (int)std::min<long>({(long)IO_THREADS, total == 1 ? 1 : 1 + total / 2,
+                                          std::max(1L, (long)std::thread::hardware_concurrency() / 2)});
+    std::vector<std::thread> crew;
+    try {
+        crew.reserve(want);
+        for (int t = 1; t < want; ++t) crew.emplace_back(work, t);
+    } catch (...) {
+        // fewer threads than wanted: those that started take all chunks
+    }
+    work(0);
+    for (std::thread &t : crew) t.join();
+    const hipError_t e = hipStreamSynchronize(c->stream);
+    io_release(b);
+    if (bad.load() != hipSuccess) return fail(std::string("field copy: ") + hipGetErrorString((hipError_t)bad.load()));
+    if (e != hipSuccess) return fail(std::string("field copy: ") + hipGetErrorString(e));
+    return 0;
+}
+
+// rows of a chunk between the pinned buffer and the caller's field
+void io_copy(const s3d_ctx *c, const IoChunk &k, double *field, double *chunk, bool out)
+{
+    double *f = field + (size_t)k.n0 * c->nel + k.e0;
+    const long rows = k.ne == c->nel ? 1 : k.nn;
+    const size_t words = (size_t)k.ne * k.nn / rows;
+    for (long r = 0; r < rows; ++r) {
+        double *a = f + r * c->nel, *b = chunk + r * words;
+        std::memcpy(out ? a : b, out ? b : a, words * sizeof(double));
+    }
+}
+
+template <typename Src>
+int io_get(s3d_ctx *c, const Src &src, double *out)
+{
+    return io_chunks(c, 1, [&](const IoChunk &k, double *chunk, hipEvent_t ev) {
+        hipLaunchKernelGGL(export_field<Src>, k.grid(), dim3(256), 0, c->stream, src, k.e0, k.ne, k.n0, k.nn, chunk);
+        hipError_t e = hipGetLastError();
+        if (e == hipSuccess) e = hipEventRecord(ev, c->stream);
+        if (e == hipSuccess) e = hipEventSynchronize(ev);
+        if (e == hipSuccess) io_copy(c, k, out, chunk, true);
+        return e;
+    });
+}
+
+template <typename Dst>
+int io_set(s3d_ctx *c, const Dst &dst, const double *in)
+{
+    return io_chunks(c, 1, [&](const IoChunk &k, double *chunk, hipEvent_t ev) {
+        hipError_t e = hipEventSynchronize(ev);   // the buffer's last chunk
+        if (e != hipSuccess) return e;
+        io_copy(c, k, const_cast<double *>(in), chunk, false);
+        hipLaunchKernelGGL(import_field<Dst>, k.grid(), dim3(256), 0, c->stream, dst, k.e0, k.ne, k.n0, k.nn, chunk);
+        e = hipGetLastError();
+        return e == hipSuccess ? hipEventRecord(ev, c->stream) : e;
+    });
+}
+
+template <int P, typename R>
+UniqueSrc<P, R> unique_src(const s3d_ctx *c, const void *v, const void *lo)
+{
+    UniqueSrc<P, R> s;
+    s.v = (decltype(s.v))((const R *)v);
+    s.lo = (decltype(s.lo))((const R *)(c->kv == 1 ? lo : nullptr));
+    s.lo16 = (decltype(s.lo16))((const bf16 *)(c->kv == 2 ? lo : nullptr));
+    s.nx = c->g.nx;
+    s.ny = c->g.ny;
+    return s;
+}
+
+template <int P, typename R>
+struct UniqueGetRun {
+    static int run(s3d_ctx *c, const void *v, const void *lo, double *out)
+    {
+        return io_get(c, unique_src<P, R>(c, v, lo), out);
+    }
+};
+
+template <int P, typename R>
+struct UniqueSetRun {
+    static int run(s3d_ctx *c, const double *in, void *v, void *lo)
+    {
+        UniqueDst<P, R> d;
+        d.v = (decltype(d.v))((R *)v);
+        d.lo = (decltype(d.lo))((R *)(c->kv == 1 ? lo : nullptr));
+        d.lo16 = (decltype(d.lo16))((bf16 *)(c->kv == 2 ? lo : nullptr));
+        d.nx = c->g.nx;
+        d.ny = c->g.ny;
+        d.nz = c->g.nz;
+        return io_set(c, d, in);
+    }
+};
+
+template <int P, typename R>
+struct CurlGetRun {
+    static int run(s3d_ctx *c, int comp, double *out)
+    {
+        CurlSrc<P, R> s;
+        s.a = curl_args<P, R>(c);
+        s.parts = (decltype(s.parts))((const double *)c->curl_parts);
+        s.comp = comp;
+        return io_get(c, s, out);
+    }
+};
+
+template <int P, typename R>
+struct GradRun {
+    static int run(s3d_ctx *c, const double *const *fw, double inc_dt)
+    {
+        GradArgs<P, R> a;
+        a.g = (decltype(a.g))((double *)c->grad_rho);
+        for (int q = 0; q < 3; ++q) a.v[q] = unique_src<P, R>(c, c->v[q], c->lo[q]);
+        a.inc_dt = inc_dt;
+        a.jac = c->jac;
+        return io_chunks(c, 3, [&](const IoChunk &k, double *chunk, hipEvent_t ev) {
+            hipError_t e = hipEventSynchronize(ev);
+            if (e != hipSuccess) return e;
+            for (int q = 0; q < 3; ++q)
+                io_copy(c, k, const_cast<double *>(fw[q]), chunk + (size_t)q * k.ne * k.nn, false);
+            hipLaunchKernelGGL((grad_rho_kernel<P, R>), k.grid(), dim3(256), 0, c->stream, a, k.e0, k.ne, k.n0, k.nn,
+                               chunk);
+            e = hipGetLastError();
+            return e == hipSuccess ? hipEventRecord(ev, c->stream) : e;
+        });
     }
 };
 
@@ -763,45 +1026,6 @@ struct CurlPartsRun {
     {
         hipLaunchKernelGGL((curl_parts_kernel<P, R>), dim3((unsigned)c->nel), dim3(64), 0, c->stream,
                            curl_args<P, R>(c), c->nel, (double *)c->curl_parts);
-        HIPCHK(hipGetLastError());
-        return 0;
-    }
-};
-
-template <int P, typename R>
-struct CurlFieldRun {
-    static int run(s3d_ctx *c, int comp, double *out)
-    {
-        hipLaunchKernelGGL((curl_field_kernel<P, R>), dim3(nblocks(c->nn, 256)), dim3(256), 0, c->stream,
-                           curl_args<P, R>(c), c->g.nz, c->nn, (const double *)c->curl_parts, comp, out);
-        HIPCHK(hipGetLastError());
-        return 0;
-    }
-};
-
-template <int P, typename R>
-struct GradRun {
-    static int run(s3d_ctx *c, const double *f, double inc_dt)
-    {
-        const long nn = c->nn;
-        hipLaunchKernelGGL((grad_rho_kernel<P, R>), dim3(nblocks(nn, 256)), dim3(256), 0, c->stream,
-                           (double *)c->grad_rho, f, f + nn, f + 2 * nn, (const R *)c->v[0],
-                           (const R *)c->v[1], (const R *)c->v[2], (const R *)lo32<R>(c, 0),
-                           (const R *)lo32<R>(c, 1), (const R *)lo32<R>(c, 2), (const bf16 *)lo16(c, 0),
-                           (const bf16 *)lo16(c, 1), (const bf16 *)lo16(c, 2), c->g.nx, c->g.ny, c->g.nz,
-                           inc_dt, c->jac);
-        HIPCHK(hipGetLastError());
-        return 0;
-    }
-};
-
-template <int P, typename R>
-struct GatherRun {
-    static int run(s3d_ctx *c, const double *src, void *dst, void *lo)
-    {
-        hipLaunchKernelGGL((gather_unique<P, R>), dim3(nblocks(c->nuniq, 256)), dim3(256), 0, c->stream,
-                           src, (R *)dst, (R *)(c->kv == 1 ? lo : nullptr), (bf16 *)(c->kv == 2 ? lo : nullptr),
-                           c->g.nx, c->g.ny, c->g.nz, c->nblk);
         HIPCHK(hipGetLastError());
         return 0;
     }
@@ -1357,6 +1581,7 @@ int s3d_create(const s3d_grid *grid, const s3d_options *opt, s3d_ctx **out)
     c->nblk = (long)(grid->nx + 1) * (grid->ny + 1) * (grid->nz + 1);
     c->nuniq = c->nblk * c->PB;
     gll_tables(c->p, c->knots, c->weights, c->dl);
+    io_live(c->dev, 1);
     *out = c;
     return 0;
 }
@@ -1384,7 +1609,7 @@ int s3d_destroy(s3d_ctx *c)
     for (int q = 0; q < 7; ++q) dfree(c->stage[q]);
     c->sig = c->sig_lo = c->mem = nullptr;   // views of the state blocks
     void *bufs[] = {c->v[0], c->v[1], c->v[2], c->lo[0], c->lo[1], c->lo[2], c->dt_inv_mm, c->blk[0], c->blk[1],
-                    c->mat, c->rho, c->ca, c->cb, c->cc, c->grad_rho, c->grad_stage, c->dgrad, c->curl_parts,
+                    c->mat, c->rho, c->ca, c->cb, c->cc, c->grad_rho, c->dgrad, c->curl_parts,
                     c->force, c->tth, c->tr, c->wdev, c->mm64, c->dpx, c->dpy, c->dpz,
                     c->d_slot, c->d_chan, c->d_coef, c->d_stf, c->d_rec_e, c->d_rec_nch,
                     c->d_rec_off, c->d_rec_ch, c->d_rec_vm, c->d_traces, c->d_rec_rot, c->d_rot_e, c->d_rot_buf};
@@ -1394,6 +1619,7 @@ int s3d_destroy(s3d_ctx *c)
     drop_graph(c);
     dfree(c->d_it);
     if (c->stream) (void)hipStreamDestroy(c->stream);
+    io_live(c->dev, -1);
     delete c;
     return 0;
 }
@@ -1437,6 +1663,7 @@ int s3d_create_shared(s3d_ctx *base, s3d_ctx **out)
     c->wdev = m->wdev; c->dpx = m->dpx; c->dpy = m->dpy; c->dpz = m->dpz;
     c->model = m;
     m->sharers++;
+    io_live(c->dev, 1);
     hipError_t e = hipStreamCreate(&c->stream);
     if (e != hipSuccess) {
         s3d_destroy(c);
@@ -1923,6 +2150,80 @@ static int mem_word(const s3d_ctx *c, int field)
     return c->nm == 5 ? 5 * (f / 6) + f % 6 : f;
 }
 
+}  // extern "C"
+
+template <typename R>
+static int get_block(s3d_ctx *c, const R *p, const R *lo, int nc, double *out)
+{
+    BlockSrc<R> s;
+    s.p = (decltype(s.p))(p);
+    s.lo = (decltype(s.lo))(lo);
+    s.nc = nc;
+    s.NP = c->NP;
+    return io_get(c, s, out);
+}
+
+// a stress component (less its compensation) or a memory variable
+template <typename R>
+static int get_state(s3d_ctx *c, int field, double *out)
+{
+    const long NP = c->NP;
+    if (field <= S3D_SZZ) {
+        const int q = field - S3D_SXX;
+        const R *sig = (const R *)c->sig + NP * q;
+        if (c->o.kahan_sigma != 2)
+            return get_block<R>(c, sig, c->sig_lo ? (const R *)c->sig_lo + NP * q : nullptr, c->ns, out);
+        PairSrc s;   // FP32 only
+        s.p = (decltype(s.p))((const float *)c->sig + NP * q);
+        s.lo = (decltype(s.lo))((const unsigned *)c->sig_lo + NP * (q / 2));
+        s.half = q % 2;
+        s.nc = c->ns;
+        s.NP = c->NP;
+        return io_get(c, s, out);
+    }
+    const R *mem = (const R *)c->mem;
+    if (c->nm == 5 && (field - S3D_MXX) % 6 == ZZ) {
+        // five-word form: zz is not stored, it is -(xx + yy)
+        const int m0 = S3D_MXX + 6 * ((field - S3D_MXX) / 6);
+        DeviatorSrc<R> s;
+        s.xx = (decltype(s.xx))(mem + NP * mem_word(c, m0 + XX));
+        s.yy = (decltype(s.yy))(mem + NP * mem_word(c, m0 + YY));
+        s.nc = c->ns;
+        s.NP = c->NP;
+        return io_get(c, s, out);
+    }
+    return get_block<R>(c, mem + NP * mem_word(c, field), nullptr, c->ns, out);
+}
+
+template <typename R>
+static int set_state(s3d_ctx *c, int field, const double *in)
+{
+    const long NP = c->NP;
+    BlockDst<R> d;
+    d.lo = nullptr;
+    d.nc = c->ns;
+    d.NP = c->NP;
+    if (field <= S3D_SZZ) {
+        const int q = field - S3D_SXX;
+        if (c->o.kahan_sigma == 2) {   // FP32 only
+            PairDst t;
+            t.p = (decltype(t.p))((float *)c->sig + NP * q);
+            t.lo = (decltype(t.lo))((unsigned *)c->sig_lo + NP * (q / 2));
+            t.half = q % 2;
+            t.nc = c->ns;
+            t.NP = c->NP;
+            return io_set(c, t, in);
+        }
+        d.p = (decltype(d.p))((R *)c->sig + NP * q);
+        if (c->sig_lo) d.lo = (decltype(d.lo))((R *)c->sig_lo + NP * q);
+    } else {
+        d.p = (decltype(d.p))((R *)c->mem + NP * mem_word(c, field));
+    }
+    return io_set(c, d, in);
+}
+
+extern "C" {
+
 int s3d_get_field(s3d_ctx *c, int field, double *out)
 {
     if (!c || !out) return fail("null argument");
@@ -1932,12 +2233,9 @@ int s3d_get_field(s3d_ctx *c, int field, double *out)
     if (field >= S3D_GRAD_RHO && field <= S3D_GRAD_CSV) {
         // grad_cs/cp/csh/csv: the reference builds them from forward strain
         // rates it never loads; they read as zero
-        if (field == S3D_GRAD_RHO && c->grad_rho) {
-            HIPCHK(hipMemcpyAsync(out, c->grad_rho, sizeof(double) * nn, hipMemcpyDeviceToHost, c->stream));
-            HIPCHK(hipStreamSynchronize(c->stream));
-        } else {
-            std::memset(out, 0, sizeof(double) * nn);
-        }
+        if (field == S3D_GRAD_RHO && c->grad_rho)
+            return get_block<double>(c, (const double *)c->grad_rho, nullptr, 1, out);
+        std::memset(out, 0, sizeof(double) * nn);
         return 0;
     }
     if (field == S3D_TAPER) {
@@ -1957,88 +2255,30 @@ int s3d_get_field(s3d_ctx *c, int field, double *out)
                             }
         return 0;
     }
-    double *buf = nullptr;
-    HIPCHK(hipMalloc(&buf, sizeof(double) * nn));
-    int rc = 0;
-    if (field >= S3D_VX && field <= S3D_VZ) {
-        rc = c->fp32 ? with_p<ExpandRun, float>(c->p, c, (const void *)c->v[field], (const void *)c->lo[field], buf)
-                     : with_p<ExpandRun, double>(c->p, c, (const void *)c->v[field], (const void *)nullptr, buf);
-    } else if (field == S3D_MM) {
-        rc = with_p<ExpandRun, double>(c->p, c, (const void *)c->mm64, (const void *)nullptr, buf);
-    } else if (field >= S3D_ROT_VX && field <= S3D_ROT_VZ) {
-        if (!c->curl_parts || c->curl_it != c->it - 1) {
-            (void)hipFree(buf);
+    if (field >= S3D_VX && field <= S3D_VZ)
+        return c->fp32 ? with_p<UniqueGetRun, float>(c->p, c, (const void *)c->v[field], (const void *)c->lo[field], out)
+                       : with_p<UniqueGetRun, double>(c->p, c, (const void *)c->v[field], (const void *)nullptr, out);
+    if (field == S3D_MM) return with_p<UniqueGetRun, double>(c->p, c, (const void *)c->mm64, (const void *)nullptr, out);
+    if (field >= S3D_ROT_VX && field <= S3D_ROT_VZ) {
+        if (!c->curl_parts || c->curl_it != c->it - 1)
             return fail("volume curl fields need s3d_capture_curl_strain just before the last step");
-        }
         const int comp = field - S3D_ROT_VX;
-        rc = c->fp32 ? with_p<CurlFieldRun, float>(c->p, c, comp, buf)
-                     : with_p<CurlFieldRun, double>(c->p, c, comp, buf);
-    } else if (field >= S3D_EXX && field <= S3D_EZZ) {
-        if (!c->dgrad) {
-            (void)hipFree(buf);
+        return c->fp32 ? with_p<CurlGetRun, float>(c->p, c, comp, out) : with_p<CurlGetRun, double>(c->p, c, comp, out);
+    }
+    if (field >= S3D_EXX && field <= S3D_EZZ) {
+        if (!c->dgrad)
             return fail("the displacement gradient is not integrated: call s3d_enable_displacement_gradient "
                         "before stepping");
-        }
-        hipLaunchKernelGGL(from_device_layout<double>, dim3(nblocks(nn, 256)), dim3(256), 0, c->stream,
-                           (const double *)c->dgrad + (long)c->NP * (field - S3D_EXX), buf, c->nel, c->NP, 6);
-    } else if (field >= S3D_MXX && field < S3D_MXX + 18 && c->mem && c->nm == 5 &&
-               (field - S3D_MXX) % 6 == ZZ) {
-        // five-word form: zz is not stored, it is -(xx + yy)
-        (void)hipFree(buf);
-        std::vector<double> xx(nn), yy(nn);
-        const int m0 = S3D_MXX + 6 * ((field - S3D_MXX) / 6);
-        if (int rc = s3d_get_field(c, m0 + XX, xx.data())) return rc;
-        if (int rc = s3d_get_field(c, m0 + YY, yy.data())) return rc;
-        for (long q = 0; q < nn; ++q) out[q] = -(xx[q] + yy[q]);
-        return 0;
-    } else if ((field >= S3D_SXX && field <= S3D_SZZ) || (field >= S3D_MXX && field < S3D_MXX + 18)) {
-        const void *src = nullptr;
-        const void *lo = nullptr;
-        const int nc = c->ns;   // components of the state block
-        if (field <= S3D_SZZ) {
-            src = (const char *)c->sig + rsize(c) * c->NP * (field - S3D_SXX);
-            if (c->sig_lo && c->o.kahan_sigma == 1) lo = (const char *)c->sig_lo + rsize(c) * c->NP * (field - S3D_SXX);
-            if (c->sig_lo && c->o.kahan_sigma == 2) lo = (const char *)c->sig_lo + 4 * c->NP * ((field - S3D_SXX) / 2);
-        } else if (c->mem) {
-            src = (const char *)c->mem + rsize(c) * c->NP * mem_word(c, field);
-        }
-        if (!src) {
-            HIPCHK(hipMemsetAsync(buf, 0, sizeof(double) * nn, c->stream));
-        } else if (c->fp32) {
-            hipLaunchKernelGGL(from_device_layout<float>, dim3(nblocks(nn, 256)), dim3(256), 0, c->stream,
-                               (const float *)src, buf, c->nel, c->NP, nc);
-            if (lo) {
-                // value = hi - lo
-                double *tmp = nullptr;
-                HIPCHK(hipMalloc(&tmp, sizeof(double) * nn));
-                if (c->o.kahan_sigma == 2)
-                    hipLaunchKernelGGL(lo_pair_from_device, dim3(nblocks(nn, 256)), dim3(256), 0, c->stream,
-                                       (const unsigned *)lo, (field - S3D_SXX) % 2, tmp, c->nel, c->NP, nc);
-                else
-                    hipLaunchKernelGGL(from_device_layout<float>, dim3(nblocks(nn, 256)), dim3(256), 0, c->stream,
-                                       (const float *)lo, tmp, c->nel, c->NP, nc);
-                std::vector<double> a(nn), b(nn);
-                HIPCHK(hipMemcpyAsync(a.data(), buf, sizeof(double) * nn, hipMemcpyDeviceToHost, c->stream));
-                HIPCHK(hipMemcpyAsync(b.data(), tmp, sizeof(double) * nn, hipMemcpyDeviceToHost, c->stream));
-                HIPCHK(hipStreamSynchronize(c->stream));
-                (void)hipFree(tmp);
-                for (long q = 0; q < nn; ++q) out[q] = a[q] - b[q];
-                (void)hipFree(buf);
-                return 0;
-            }
-        } else {
-            hipLaunchKernelGGL(from_device_layout<double>, dim3(nblocks(nn, 256)), dim3(256), 0, c->stream,
-                               (const double *)src, buf, c->nel, c->NP, nc);
-        }
-    } else {
-        (void)hipFree(buf);
-        return fail("unknown field id " + std::to_string(field));
+        return get_block<double>(c, (const double *)c->dgrad + (long)c->NP * (field - S3D_EXX), nullptr, 6, out);
     }
-    if (rc) { (void)hipFree(buf); return rc; }
-    HIPCHK(hipMemcpyAsync(out, buf, sizeof(double) * nn, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    (void)hipFree(buf);
-    return 0;
+    if ((field >= S3D_SXX && field <= S3D_SZZ) || (field >= S3D_MXX && field < S3D_MXX + 18)) {
+        if (field > S3D_SZZ && !c->mem) {
+            std::memset(out, 0, sizeof(double) * nn);
+            return 0;
+        }
+        return c->fp32 ? get_state<float>(c, field, out) : get_state<double>(c, field, out);
+    }
+    return fail("unknown field id " + std::to_string(field));
 }
 
 int s3d_set_field(s3d_ctx *c, int field, const double *in)
@@ -2047,50 +2287,17 @@ int s3d_set_field(s3d_ctx *c, int field, const double *in)
     if (!c->inited) return fail("s3d_init first");
     HIPCHK(hipSetDevice(c->dev));
     c->fields_set = true;
-    const long nn = c->nn;
-    double *buf = nullptr;
-    HIPCHK(hipMalloc(&buf, sizeof(double) * nn));
-    HIPCHK(hipMemcpyAsync(buf, in, sizeof(double) * nn, hipMemcpyHostToDevice, c->stream));
-    int rc = 0;
-    if (field >= S3D_VX && field <= S3D_VZ) {
-        rc = c->fp32 ? with_p<GatherRun, float>(c->p, c, (const double *)buf, c->v[field], c->lo[field])
-                     : with_p<GatherRun, double>(c->p, c, (const double *)buf, c->v[field], (void *)nullptr);
-    } else if ((field >= S3D_SXX && field <= S3D_SZZ) || (field >= S3D_MXX && field < S3D_MXX + 18)) {
-        void *dst = nullptr;
-        const int nc = c->ns;   // components of the state block
-        if (field <= S3D_SZZ) {
-            dst = (char *)c->sig + rsize(c) * c->NP * (field - S3D_SXX);
-            if (c->sig_lo && c->o.kahan_sigma == 1)
-                hipLaunchKernelGGL(clear_component<float>, dim3(nblocks(nn, 256)), dim3(256), 0, c->stream,
-                                   (float *)c->sig_lo + c->NP * (field - S3D_SXX), c->nel, c->NP, nc);
-            if (c->sig_lo && c->o.kahan_sigma == 2)
-                hipLaunchKernelGGL(lo_pair_clear, dim3(nblocks(nn, 256)), dim3(256), 0, c->stream,
-                                   (unsigned *)c->sig_lo + c->NP * ((field - S3D_SXX) / 2), (field - S3D_SXX) % 2,
-                                   c->nel, c->NP, nc);
-        } else if (c->mem && c->nm == 5 && (field - S3D_MXX) % 6 == ZZ) {
-            rc = fail("with five memory words per mechanism the zz memory variables are -(xx + yy) "
-                      "and cannot be set");
-        } else if (c->mem) {
-            dst = (char *)c->mem + rsize(c) * c->NP * mem_word(c, field);
-        } else {
-            rc = fail("memory variables exist only for a visco-elastic model");
-        }
-        if (dst) {
-            if (c->fp32)
-                hipLaunchKernelGGL(to_device_layout<float>, dim3(nblocks(nn, 256)), dim3(256), 0, c->stream,
-                                   (const double *)buf, (float *)dst, c->nel, c->NP, nc);
-            else
-                hipLaunchKernelGGL(to_device_layout<double>, dim3(nblocks(nn, 256)), dim3(256), 0, c->stream,
-                                   (const double *)buf, (double *)dst, c->nel, c->NP, nc);
-        }
-    } else {
-        rc = fail("field " + std::to_string(field) + " cannot be set");
+    if (field >= S3D_VX && field <= S3D_VZ)
+        return c->fp32 ? with_p<UniqueSetRun, float>(c->p, c, in, c->v[field], c->lo[field])
+                       : with_p<UniqueSetRun, double>(c->p, c, in, c->v[field], (void *)nullptr);
+    if ((field >= S3D_SXX && field <= S3D_SZZ) || (field >= S3D_MXX && field < S3D_MXX + 18)) {
+        if (field > S3D_SZZ && !c->mem) return fail("memory variables exist only for a visco-elastic model");
+        if (field > S3D_SZZ && c->nm == 5 && (field - S3D_MXX) % 6 == ZZ)
+            return fail("with five memory words per mechanism the zz memory variables are -(xx + yy) "
+                        "and cannot be set");
+        return c->fp32 ? set_state<float>(c, field, in) : set_state<double>(c, field, in);
     }
-    hipError_t e = hipStreamSynchronize(c->stream);
-    (void)hipFree(buf);
-    if (rc) return rc;
-    if (e != hipSuccess) return fail(std::string("set_field: ") + hipGetErrorString(e));
-    return 0;
+    return fail("field " + std::to_string(field) + " cannot be set");
 }
 
 int s3d_grad_add(s3d_ctx *c, const double *vx_fw, const double *vy_fw, const double *vz_fw, int increment)
@@ -2099,26 +2306,13 @@ int s3d_grad_add(s3d_ctx *c, const double *vx_fw, const double *vy_fw, const dou
     if (!c->inited) return fail("s3d_init first");
     if (increment == 0) return fail("grad_add: increment must be nonzero");
     HIPCHK(hipSetDevice(c->dev));
-    const long nn = c->nn;
-    if (!c->grad_rho && dalloc(c, &c->grad_rho, sizeof(double) * nn)) return 1;
-    // the snapshot staging buffer is kept for the next saved step
-    if (!c->grad_stage && dalloc(c, &c->grad_stage, sizeof(double) * 3 * nn, false)) return 1;
-    double *f = (double *)c->grad_stage;
-    const double *src[3] = {vx_fw, vy_fw, vz_fw};
-    int rc = 0;
-    for (int q = 0; q < 3 && !rc; ++q)
-        if (hipMemcpyAsync(f + q * nn, src[q], sizeof(double) * nn, hipMemcpyHostToDevice, c->stream) != hipSuccess)
-            rc = fail("grad_add: upload failed");
+    if (!c->grad_rho && dalloc(c, &c->grad_rho, sizeof(double) * c->nn)) return 1;
+    const double *fw[3] = {vx_fw, vy_fw, vz_fw};
     // increment*dt as the reference forms it, before the product and the
     // division by J
     const double inc_dt = (double)increment * c->g.dt;
-    if (!rc)
-        rc = c->fp32 ? with_p<GradRun, float>(c->p, c, (const double *)f, inc_dt)
-                     : with_p<GradRun, double>(c->p, c, (const double *)f, inc_dt);
-    hipError_t e = hipStreamSynchronize(c->stream);
-    if (rc) return rc;
-    if (e != hipSuccess) return fail(std::string("grad_add: ") + hipGetErrorString(e));
-    return 0;
+    return c->fp32 ? with_p<GradRun, float>(c->p, c, (const double *const *)fw, inc_dt)
+                   : with_p<GradRun, double>(c->p, c, (const double *const *)fw, inc_dt);
 }
 
 int s3d_enable_displacement_gradient(s3d_ctx *c)

@@ -26,13 +26,6 @@
 
 namespace s3d {
 
-// vel_lo for plain pointers (the set-up and field kernels)
-template <typename R>
-__device__ __forceinline__ double lo_at(const R *l, const bf16 *h, long u)
-{
-    return l ? (double)l[u] : h ? (double)(float)h[u] : 0.0;
-}
-
 // ---------------------------------------------------------------------------
 // node kernel: assembly, 1/M, velocity integration, taper
 // ---------------------------------------------------------------------------
@@ -388,29 +381,28 @@ __global__ void __launch_bounds__(64) curl_parts_kernel(const CurlArgs<R> a, lon
     }
 }
 
-// Volume curl fields, second half: rot_v{x,y,z} (comp 0, 1, 2) of every
-// element-local node from the stored parts and the current velocity, in the
-// reference's 6-D layout out[ex + nx (ey + ny (ez + nz (i + P1 (j + P1 k))))].
+// Volume curl fields, second half: rot_v{x,y,z} (comp 0, 1, 2) of node n of
+// element e from the stored parts and the current velocity (a source of
+// export_field).
 template <int P, typename R>
-__global__ void __launch_bounds__(256) curl_field_kernel(const CurlArgs<R> a, int nz, long nn,
-                                                         const double *parts, int comp, double *out)
-{
-    constexpr int P1 = P + 1, NP = P1 * P1 * P1;
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nn) return;
-    const long e = t / NP;
-    const int n = (int)(t - e * NP);
-    const int ex = (int)(e % a.nx), ey = (int)((e / a.nx) % a.ny), ez = (int)(e / ((long)a.nx * a.ny));
-    const int i = n % P1, j = (n / P1) % P1, k = n / (P1 * P1);
-    double part[6];
+struct CurlSrc {
+    CurlArgs<R> a;
+    gptr<const double> parts;
+    int comp;
+    __device__ double operator()(long e, int n) const
+    {
+        constexpr int P1 = P + 1, NP = P1 * P1 * P1;
+        const int ex = (int)(e % a.nx), ey = (int)((e / a.nx) % a.ny), ez = (int)(e / ((long)a.nx * a.ny));
+        const int i = n % P1, j = (n / P1) % P1, k = n / (P1 * P1);
+        double part[6];
 #pragma unroll
-    for (int c = 0; c < 6; ++c) part[c] = parts[(e * 6 + c) * NP + n];
-    const long u = unique_index<P>(ex, ey, ez, i, j, k, a.nx, a.ny);
-    const double vxn = curl_vel(a.vx, a.lx, a.hx, u), vyn = curl_vel(a.vy, a.ly, a.hy, u);
-    const double r = a.tr[ez * P1 + k].r, st = a.tth[ex * P1 + i].sin_t, ct = a.tth[ex * P1 + i].cot;
-    const long o = ex + (long)a.nx * (ey + (long)a.ny * (ez + (long)nz * (i + (long)P1 * (j + (long)P1 * k))));
-    out[o] = curl_formula(comp, part, vxn, vyn, r, r * st, ct, st);
-}
+        for (int c = 0; c < 6; ++c) part[c] = parts[(e * 6 + c) * NP + n];
+        const long u = unique_index<P>(ex, ey, ez, i, j, k, a.nx, a.ny);
+        const double vxn = curl_vel(a.vx, a.lx, a.hx, u), vyn = curl_vel(a.vy, a.ly, a.hy, u);
+        const double r = a.tr[ez * P1 + k].r, st = a.tth[ex * P1 + i].sin_t, ct = a.tth[ex * P1 + i].cot;
+        return curl_formula(comp, part, vxn, vyn, r, r * st, ct, st);
+    }
+};
 
 template <int P, typename R>
 __global__ void __launch_bounds__(64) record_kernel(const RecArgs<R> a)
@@ -443,126 +435,188 @@ __global__ void __launch_bounds__(64) advance_many_kernel(int *const *its, int n
 // setup and I/O kernels
 // ---------------------------------------------------------------------------
 
-// Conversions between the reference layout [n][e] (FP64) and one component
-// of an element-major block field of nc components (dst/src point at the
-// component's first entry; element e's entries start at e * nc * NP).
+// Fields to and from the host. The host side is the reference layout [n][e]
+// (FP64, e fastest), the device fields are element-major or on unique nodes,
+// so both directions transpose a tile of IO_E elements x IO_N nodes in LDS:
+// device memory is read and written along the nodes of an element, the host
+// image along the elements. The host image is one chunk of the field in
+// pinned host memory (nodes n0 .. n0+nn-1, elements e0 .. e0+ne-1,
+// chunk[(n - n0) * ne + (e - e0)]), which the kernels read and write directly,
+// 256 B per half wave: no device copy of the field, no separate transfer. What
+// bounds them is the host link. (With one lane per value in host order and a
+// device buffer, at 96x96x48, order 4, the conversion alone took 1.0 ms for a
+// stress component, 2.1 ms for a velocity component.)
+constexpr int IO_E = 32, IO_N = 64;
+
+// Sources: value of node n of element e.
+// One component of an element-major block of nc components, less its FP32
+// compensation words (lo null: none).
 template <typename R>
-__global__ void to_device_layout(const double *src, R *dst, long nel, int NP, int nc)
-{
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nel * NP) return;
-    long e = t / NP;
-    int n = (int)(t - e * NP);
-    dst[e * nc * NP + n] = (R)src[(long)n * nel + e];
-}
+struct BlockSrc {
+    gptr<const R> p, lo;
+    int nc, NP;
+    __device__ double operator()(long e, int n) const
+    {
+        const long a = e * nc * NP + n;
+        return lo ? (double)p[a] - (double)lo[a] : (double)p[a];
+    }
+};
 
+// The same with BF16 compensation words in pairs.
+struct PairSrc {
+    gptr<const float> p;
+    gptr<const unsigned> lo;
+    int half, nc, NP;
+    __device__ double operator()(long e, int n) const
+    {
+        const long a = e * nc * NP + n;
+        const unsigned w = lo[a];
+        return (double)p[a] - (double)(half ? bf16_hi(w) : bf16_lo(w));
+    }
+};
+
+// zz of a deviatoric memory variable
 template <typename R>
-__global__ void from_device_layout(const R *src, double *dst, long nel, int NP, int nc)
+struct DeviatorSrc {
+    gptr<const R> xx, yy;
+    int nc, NP;
+    __device__ double operator()(long e, int n) const
+    {
+        const long a = e * nc * NP + n;
+        return -((double)xx[a] + (double)yy[a]);
+    }
+};
+
+template <int P, typename R>
+struct UniqueSrc {
+    gptr<const R> v, lo;
+    gptr<const bf16> lo16;
+    int nx, ny;
+    __device__ double operator()(long e, int n) const
+    {
+        constexpr int P1 = P + 1;
+        const int i = n % P1, j = (n / P1) % P1, k = n / (P1 * P1);
+        const int ex = (int)(e % nx), ey = (int)((e / nx) % ny), ez = (int)(e / ((long)nx * ny));
+        const long u = unique_index<P>(ex, ey, ez, i, j, k, nx, ny);
+        return (double)v[u] - vel_lo(lo, lo16, u);
+    }
+};
+
+template <typename Src>
+__global__ void __launch_bounds__(256) export_field(const Src src, long e0, int ne, int n0, int nn, double *chunk)
 {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nel * NP) return;
-    long n = t / nel;
-    long e = t - n * nel;
-    dst[t] = (double)src[e * nc * NP + n];
+    __shared__ double tile[IO_N][IO_E + 1];
+    const int eb = blockIdx.x * IO_E, nb = blockIdx.y * IO_N;
+    const int l = threadIdx.x & 63;
+#pragma unroll
+    for (int q = threadIdx.x >> 6; q < IO_E; q += 4)
+        if (eb + q < ne && nb + l < nn) tile[l][q] = src(e0 + eb + q, n0 + nb + l);
+    __syncthreads();
+    const int e = eb + (threadIdx.x & 31);
+#pragma unroll
+    for (int q = threadIdx.x >> 5; q < IO_N; q += 8)
+        if (e < ne && nb + q < nn) chunk[(long)(nb + q) * ne + e] = tile[q][threadIdx.x & 31];
 }
 
+// Destinations: store the value of node n of element e.
+// One component of an element-major block of nc components; its FP32
+// compensation word (lo not null) becomes zero.
 template <typename R>
-__global__ void clear_component(R *p, long nel, int NP, int nc)
-{
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nel * NP) return;
-    long e = t / NP;
-    int n = (int)(t - e * NP);
-    p[e * nc * NP + n] = R(0);
-}
+struct BlockDst {
+    gptr<R> p, lo;
+    int nc, NP;
+    __device__ void operator()(long e, int n, double x) const
+    {
+        const long a = e * nc * NP + n;
+        p[a] = (R)x;
+        if (lo) lo[a] = R(0);
+    }
+};
 
-// one half of a packed BF16 stress compensation component of a block of nc
-// -> reference layout
-__global__ void lo_pair_from_device(const unsigned *src, int half, double *dst, long nel, int NP, int nc)
-{
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nel * NP) return;
-    long n = t / nel;
-    long e = t - n * nel;
-    const unsigned w = src[e * nc * NP + n];
-    dst[t] = (double)(half ? bf16_hi(w) : bf16_lo(w));
-}
+// The same with BF16 compensation words in pairs: the component's half.
+struct PairDst {
+    gptr<float> p;
+    gptr<unsigned> lo;
+    int half, nc, NP;
+    __device__ void operator()(long e, int n, double x) const
+    {
+        const long a = e * nc * NP + n;
+        p[a] = (float)x;
+        lo[a] &= half ? 0x0000ffffu : 0xffff0000u;
+    }
+};
 
-// clear one half of one packed BF16 stress compensation component of a block
-// of nc
-__global__ void lo_pair_clear(unsigned *p, int half, long nel, int NP, int nc)
+// A unique-node field takes the owner element's copy of a node: the element
+// whose block holds it, the last element on the far domain faces.
+template <int P, typename R>
+struct UniqueDst {
+    gptr<R> v, lo;
+    gptr<bf16> lo16;
+    int nx, ny, nz;
+    __device__ void operator()(long e, int n, double x) const
+    {
+        constexpr int P1 = P + 1;
+        const int i = n % P1, j = (n / P1) % P1, k = n / (P1 * P1);
+        const int ex = (int)(e % nx), ey = (int)((e / nx) % ny), ez = (int)(e / ((long)nx * ny));
+        if ((i == P && ex < nx - 1) || (j == P && ey < ny - 1) || (k == P && ez < nz - 1)) return;
+        const long u = unique_index<P>(ex, ey, ez, i, j, k, nx, ny);
+        v[u] = (R)x;
+        if (lo) lo[u] = (R)(x - (double)(R)x) * R(-1);
+        if (lo16) lo16[u] = (bf16)(float)(-(x - (double)(R)x));
+    }
+};
+
+template <typename Dst>
+__global__ void __launch_bounds__(256) import_field(const Dst dst, long e0, int ne, int n0, int nn, const double *chunk)
 {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nel * NP) return;
-    long e = t / NP;
-    int n = (int)(t - e * NP);
-    p[e * nc * NP + n] &= half ? 0x0000ffffu : 0xffff0000u;
+    __shared__ double tile[IO_N][IO_E + 1];
+    const int eb = blockIdx.x * IO_E, nb = blockIdx.y * IO_N;
+    const int e = eb + (threadIdx.x & 31);
+#pragma unroll
+    for (int q = threadIdx.x >> 5; q < IO_N; q += 8)
+        if (e < ne && nb + q < nn) tile[q][threadIdx.x & 31] = chunk[(long)(nb + q) * ne + e];
+    __syncthreads();
+    const int l = threadIdx.x & 63;
+#pragma unroll
+    for (int q = threadIdx.x >> 6; q < IO_E; q += 4)
+        if (eb + q < ne && nb + l < nn) dst(e0 + eb + q, n0 + nb + l, tile[l][q]);
 }
 
 // Adjoint density sensitivity (reference ses3d_grad,
-// src/SOURCE/ses3d_grad.F90:212-213), all arrays in the reference layout
-// [n][e]: g += inc_dt * (fx*vx + fy*vy + fz*vz) / jac, the velocity (hi - lo)
-// gathered from the unique nodes.
+// src/SOURCE/ses3d_grad.F90:212-213): g += inc_dt * (fx*vx + fy*vy + fz*vz) / jac
+// for the nodes and elements of one chunk of the forward snapshot in pinned
+// host memory (three components, see import_field), the velocity (hi - lo)
+// gathered from the unique nodes, g element-major [e][NP].
 template <int P, typename R>
-__global__ void grad_rho_kernel(double *g, const double *fx, const double *fy, const double *fz,
-                                const R *vx, const R *vy, const R *vz, const R *lx, const R *ly,
-                                const R *lz, const bf16 *hx, const bf16 *hy, const bf16 *hz,
-                                int nx, int ny, int nz, double inc_dt, double jac)
-{
-    constexpr int P1 = P + 1, NP = P1 * P1 * P1;
-    const long nel = (long)nx * ny * nz;
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nel * NP) return;
-    long n = t / nel;
-    long e = t - n * nel;
-    int i = (int)(n % P1), j = (int)((n / P1) % P1), k = (int)(n / (P1 * P1));
-    int ex = (int)(e % nx), ey = (int)((e / nx) % ny), ez = (int)(e / ((long)nx * ny));
-    long u = unique_index<P>(ex, ey, ez, i, j, k, nx, ny);
-    const double ax = (double)vx[u] - lo_at(lx, hx, u);
-    const double ay = (double)vy[u] - lo_at(ly, hy, u);
-    const double az = (double)vz[u] - lo_at(lz, hz, u);
-    g[t] = g[t] + inc_dt * ((fx[t] * ax + fy[t] * ay) + fz[t] * az) / jac;
-}
+struct GradArgs {
+    gptr<double> g;
+    UniqueSrc<P, R> v[3];
+    double inc_dt, jac;
+};
 
-// unique-node field -> reference layout (every copy)
 template <int P, typename R>
-__global__ void expand_unique(const R *src, const R *lo, const bf16 *lo16, double *dst, int nx, int ny, int nz)
+__global__ void __launch_bounds__(256) grad_rho_kernel(const GradArgs<P, R> a, long e0, int ne, int n0, int nn,
+                                                       const double *chunk)
 {
-    constexpr int P1 = P + 1, NP = P1 * P1 * P1;
-    const long nel = (long)nx * ny * nz;
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nel * NP) return;
-    long n = t / nel;
-    long e = t - n * nel;
-    int i = (int)(n % P1), j = (int)((n / P1) % P1), k = (int)(n / (P1 * P1));
-    int ex = (int)(e % nx), ey = (int)((e / nx) % ny), ez = (int)(e / ((long)nx * ny));
-    long u = unique_index<P>(ex, ey, ez, i, j, k, nx, ny);
-    dst[t] = (double)src[u] - lo_at(lo, lo16, u);
-}
-
-// reference layout -> unique-node field, taking the owner element's copy
-template <int P, typename R>
-__global__ void gather_unique(const double *src, R *dst, R *lo, bf16 *lo16, int nx, int ny, int nz, long nblk)
-{
-    constexpr int P1 = P + 1, PB = P * P * P;
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    long b = t / PB;
-    int o = (int)(t - b * PB);
-    if (b >= nblk) return;
-    int li = o % P, lj = (o / P) % P, lk = o / (P * P);
-    int nbx = nx + 1, nby = ny + 1;
-    int bx = (int)(b % nbx), by = (int)((b / nbx) % nby), bz = (int)(b / ((long)nbx * nby));
-    if ((bx == nx && li) || (by == ny && lj) || (bz == nz && lk)) return;
-    int ex = bx < nx ? bx : nx - 1, i = bx < nx ? li : P;
-    int ey = by < ny ? by : ny - 1, j = by < ny ? lj : P;
-    int ez = bz < nz ? bz : nz - 1, k = bz < nz ? lk : P;
-    long nel = (long)nx * ny * nz;
-    long e = ex + (long)nx * (ey + (long)ny * ez);
-    int n = i + P1 * (j + P1 * k);
-    double v = src[(long)n * nel + e];
-    dst[t] = (R)v;
-    if (lo) lo[t] = (R)(v - (double)(R)v) * R(-1);
-    if (lo16) lo16[t] = (bf16)(float)(-(v - (double)(R)v));
+    constexpr int NP = (P + 1) * (P + 1) * (P + 1);
+    __shared__ double tile[3][IO_N][IO_E + 1];
+    const int eb = blockIdx.x * IO_E, nb = blockIdx.y * IO_N;
+    const int el = eb + (threadIdx.x & 31);
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int q = threadIdx.x >> 5; q < IO_N; q += 8)
+            if (el < ne && nb + q < nn)
+                tile[c][q][threadIdx.x & 31] = chunk[((long)c * nn + nb + q) * ne + el];
+    __syncthreads();
+    const int l = threadIdx.x & 63;
+    for (int q = threadIdx.x >> 6; q < IO_E; q += 4)
+        if (eb + q < ne && nb + l < nn) {
+            const long e = e0 + eb + q;
+            const int n = n0 + nb + l;
+            const double ax = a.v[0](e, n), ay = a.v[1](e, n), az = a.v[2](e, n);
+            a.g[e * NP + n] = a.g[e * NP + n] +
+                              a.inc_dt * ((tile[0][l][q] * ax + tile[1][l][q] * ay) + tile[2][l][q] * az) / a.jac;
+        }
 }
 
 // FP64 -> storage precision (BF16 through the nearest float)
