@@ -332,8 +332,9 @@ int s3d_device_bytes(s3d_ctx *ctx, double *bytes);
 
 /* Batches: several initialised simulations on one device advance together.
  * Every step runs, for all members with the same GLL order / precision /
- * visco / compensation, ONE element kernel, ONE node kernel and ONE receiver
- * kernel (workgroups partitioned across members), and chunks of steps replay
+ * visco / compensation, ONE element kernel (which also records the receivers
+ * of the step before) and ONE node kernel (workgroups partitioned across
+ * members), and chunks of steps replay
  * one captured hipGraph. Members keep their own state, sources, receivers
  * and step counters, and may differ in mesh size and GLL order. No
  * counterpart in the reference, which runs one event per process group;

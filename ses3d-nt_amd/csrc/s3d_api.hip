@@ -206,6 +206,7 @@ struct s3d_ctx {
     // traced at rows rec_off[r] + q of the trace buffer [channels][nt]
     std::vector<int> rec_e, rec_nch, rec_off, rec_ch;
     std::vector<double> rec_vm;
+    bool rec_pressure = false;   // some receiver records the pressure
     bool rec_dirty = false;
     int *d_rec_e = nullptr, *d_rec_nch = nullptr, *d_rec_off = nullptr, *d_rec_ch = nullptr;
     double *d_rec_vm = nullptr, *d_traces = nullptr;
@@ -216,7 +217,7 @@ struct s3d_ctx {
     double *d_rot_buf = nullptr;
     int nrec_dev = 0;
     int it = 0;
-    int *d_it = nullptr;       // device copy of it, advanced by advance_kernel
+    int *d_it = nullptr;       // device copy of it, advanced by the node kernel
     // captured chunk of steps (hipGraph), one per starting state block
     hipGraph_t graph[2] = {nullptr, nullptr};
     hipGraphExec_t graph_exec[2] = {nullptr, nullptr};
@@ -442,6 +443,7 @@ NodeArgs<R> node_args(s3d_ctx *c)
     a.px = (decltype(a.px))(c->dpx); a.py = (decltype(a.py))(c->dpy); a.pz = (decltype(a.pz))(c->dpz);
     a.alpha = c->g.taper_slope;
     a.taper_on = c->g.taper_width > 0;
+    a.it_dev = (decltype(a.it_dev))(c->d_it);
     return a;
 }
 
@@ -449,6 +451,8 @@ template <typename R>
 RecArgs<R> rec_args(s3d_ctx *c)
 {
     RecArgs<R> a;
+    a.n = c->nrec_dev;
+    a.pressure = c->rec_pressure;
     a.nx = c->g.nx; a.ny = c->g.ny; a.nel = (int)c->nel; a.nt = c->g.nt;
     a.vx = (decltype(a.vx))((const R *)c->v[0]); a.vy = (decltype(a.vy))((const R *)c->v[1]); a.vz = (decltype(a.vz))((const R *)c->v[2]);
     a.lx = (decltype(a.lx))(lo32<R>(c, 0)); a.ly = (decltype(a.ly))(lo32<R>(c, 1)); a.lz = (decltype(a.lz))(lo32<R>(c, 2));
@@ -483,7 +487,7 @@ void ev_end(s3d_ctx *c, int k) { ev_begin(c, k); }
 // One element-kernel launch; the instantiation (tile, memory words, stress
 // compensation, kernel variant, BF16 statics) is chosen in s3d_elem.hip.
 template <int P, typename R>
-int launch_elem(s3d_ctx *c, const ElemArgs<R> &ea, hipStream_t st, int epb)
+int launch_elem(s3d_ctx *c, const ElemArgs<R> &ea, const RecArgs<R> &ra, hipStream_t st, int epb)
 {
     ElemLaunch l;
     l.nel = c->nel;
@@ -492,7 +496,7 @@ int launch_elem(s3d_ctx *c, const ElemArgs<R> &ea, hipStream_t st, int epb)
     l.ll = kernel_variant(c);
     l.bf16_static = c->o.bf16_static;
     l.epb = epb;
-    const hipError_t e = launch_elem_kernel<P, R>(l, ea, st);
+    const hipError_t e = launch_elem_kernel<P, R>(l, ea, ra, st);
     if (e != hipSuccess) return fail(std::string("element kernel launch: ") + hipGetErrorString(e));
     return 0;
 }
@@ -530,10 +534,12 @@ int autotune_p(s3d_ctx *c, int *tile_out, double *ms_out)
                 c->lds_layout = ll == 1 ? 1 : 0;
                 c->early_stores = ll == 2;
                 ElemArgs<R> ea = elem_args<P, R>(c);
-                if (int rc = launch_elem<P, R>(c, ea, c->stream, tile)) return rc;   // warm-up
+                RecArgs<R> none = rec_args<R>(c);
+                none.n = 0;
+                if (int rc = launch_elem<P, R>(c, ea, none, c->stream, tile)) return rc;   // warm-up
                 HIPCHK(hipEventRecord(e0, c->stream));
                 for (int r = 0; r < 3; ++r)
-                    if (int rc = launch_elem<P, R>(c, ea, c->stream, tile)) return rc;
+                    if (int rc = launch_elem<P, R>(c, ea, none, c->stream, tile)) return rc;
                 HIPCHK(hipEventRecord(e1, c->stream));
                 HIPCHK(hipEventSynchronize(e1));
                 float ms = 0.f;
@@ -579,9 +585,22 @@ CurlArgs<R> curl_args(s3d_ctx *c)
     return a;
 }
 
-template <int P, typename R>
-int launch_step(s3d_ctx *c)
+// Whether the receivers of a step can ride in the next step's element kernel:
+// it reads the velocity and the stress block as that step left them. Not with
+// curl channels (their strain parts are renewed before that kernel), not when
+// it overwrites a stress block that a pressure channel reads, and not while
+// the kernels are timed one by one.
+bool receivers_ride(const s3d_ctx *c)
 {
+    return c->nrec_dev > 0 && c->nrot == 0 && (c->nbuf == 2 || !c->rec_pressure) && !c->timing;
+}
+
+// One step; first and last: of one call or of one captured chunk, at whose
+// ends every sample is recorded.
+template <int P, typename R>
+int launch_step(s3d_ctx *c, bool first, bool last)
+{
+    const bool ride = receivers_ride(c);
     if (c->nrot > 0) {
         // before the node kernel: the curl channels use the start velocity
         hipLaunchKernelGGL((curl_strain_kernel<P, R>), dim3(c->nrot), dim3(64), 0, c->stream,
@@ -589,8 +608,10 @@ int launch_step(s3d_ctx *c)
         HIPCHK(hipGetLastError());
     }
     ElemArgs<R> ea = elem_args<P, R>(c);
+    RecArgs<R> prev = rec_args<R>(c);   // the step before: c->sig is still its stress
+    if (!ride || first) prev.n = 0;
     ev_begin(c, 0);
-    if (int rc = launch_elem<P, R>(c, ea, c->stream, c->epb)) return rc;
+    if (int rc = launch_elem<P, R>(c, ea, prev, c->stream, c->epb)) return rc;
     ev_end(c, 0);
     advance_state(c);   // the receivers read the stress this step wrote
     NodeArgs<R> na = node_args<P, R>(c);
@@ -604,33 +625,34 @@ int launch_step(s3d_ctx *c)
         hipLaunchKernelGGL((node_kernel<P, R, 0>), dim3(gn), dim3(256), 0, c->stream, na);
     ev_end(c, 1);
     HIPCHK(hipGetLastError());
-    if (c->nrec_dev > 0) {
+    if (c->nrec_dev > 0 && (last || !ride)) {
         ev_begin(c, 2);
         hipLaunchKernelGGL((record_kernel<P, R>), dim3(c->nrec_dev), dim3(64), 0, c->stream,
                            rec_args<R>(c));
         ev_end(c, 2);
         HIPCHK(hipGetLastError());
     }
-    hipLaunchKernelGGL(advance_kernel, dim3(1), dim3(64), 0, c->stream, c->d_it);
-    HIPCHK(hipGetLastError());
     return 0;
 }
 
 template <typename R>
-int dispatch_step(s3d_ctx *c)
+int dispatch_step(s3d_ctx *c, bool first, bool last)
 {
     switch (c->p) {
-    case 2: return launch_step<2, R>(c);
-    case 3: return launch_step<3, R>(c);
-    case 4: return launch_step<4, R>(c);
-    case 5: return launch_step<5, R>(c);
-    case 6: return launch_step<6, R>(c);
-    case 7: return launch_step<7, R>(c);
+    case 2: return launch_step<2, R>(c, first, last);
+    case 3: return launch_step<3, R>(c, first, last);
+    case 4: return launch_step<4, R>(c, first, last);
+    case 5: return launch_step<5, R>(c, first, last);
+    case 6: return launch_step<6, R>(c, first, last);
+    case 7: return launch_step<7, R>(c, first, last);
     default: return fail("unsupported lpd");
     }
 }
 
-int launch_one(s3d_ctx *c) { return c->fp32 ? dispatch_step<float>(c) : dispatch_step<double>(c); }
+int launch_one(s3d_ctx *c, bool first, bool last)
+{
+    return c->fp32 ? dispatch_step<float>(c, first, last) : dispatch_step<double>(c, first, last);
+}
 
 void drop_graph_slot(s3d_ctx *c, int k)
 {
@@ -658,7 +680,7 @@ int capture_graph(s3d_ctx *c, int chunk)
     drop_graph_slot(c, k);
     HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     int rc = 0;
-    for (int s = 0; s < chunk && rc == 0; ++s) rc = launch_one(c);
+    for (int s = 0; s < chunk && rc == 0; ++s) rc = launch_one(c, s == 0, s == chunk - 1);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(c->stream, &g);
     if (rc) {
@@ -1189,8 +1211,8 @@ int upload_receivers(s3d_ctx *c)
 // Batches: simulations of one device advanced together. Simulations with the
 // same (order, precision, memory-variable form, compensation) form a group;
 // each group costs
-// one element, one node and one receiver launch per step, with per-simulation
-// arguments in device arrays and workgroups partitioned by prefix sums.
+// one element and one node launch per step, with per-simulation arguments in
+// device arrays and workgroups partitioned by prefix sums.
 // ---------------------------------------------------------------------------
 struct BatchGroup {
     int p = 0;
@@ -1210,6 +1232,7 @@ struct BatchGroup {
     // per workgroup of each batched launch: (simulation, its workgroup index)
     int2 *d_eown = nullptr, *d_nown = nullptr, *d_rown = nullptr;
     int ewg = 0, nwg = 0, rwg = 0;
+    bool ride = false;          // receivers_ride for every member that has receivers
 };
 
 struct s3d_batch {
@@ -1217,7 +1240,6 @@ struct s3d_batch {
     std::vector<BatchGroup> groups;
     int dev = 0;
     hipStream_t stream = nullptr;
-    int **d_its = nullptr;
     bool built = false;
     // captured chunk of steps, one per phase (see BatchGroup)
     hipGraph_t graph[2] = {nullptr, nullptr};
@@ -1311,15 +1333,20 @@ int batch_build_group(BatchGroup &G)
 }
 
 template <int P, typename R>
-int batch_launch_group(const BatchGroup &G, hipStream_t st)
+int batch_launch_group(const BatchGroup &G, bool first, hipStream_t st)
 {
+    const size_t n = G.sims.size();
     ElemBatchLaunch l;
+    // the receivers of the step before, as it left the velocity and stress
+    l.nrec = G.ride && !first ? G.rwg : 0;
+    l.recs = (const RecArgs<R> *)G.d_rargs + (size_t)(G.phase ^ 1) * n;
+    l.rown = G.d_rown;
     l.vm = G.vm;
     l.ks = G.ks;
     l.ll = G.ll;
     l.epb = G.epb;
     l.nwg = (unsigned)G.ewg;
-    l.args = (const ElemArgs<R> *)G.d_eargs + (size_t)G.phase * G.sims.size();
+    l.args = (const ElemArgs<R> *)G.d_eargs + (size_t)G.phase * n;
     l.own = (const int2 *)G.d_eown;
     const hipError_t e = launch_elem_batch<P, R>(l, st);
     if (e != hipSuccess) return fail(std::string("batched element kernel launch: ") + hipGetErrorString(e));
@@ -1327,7 +1354,7 @@ int batch_launch_group(const BatchGroup &G, hipStream_t st)
 }
 
 template <int P, typename R>
-int batch_launch_node(const BatchGroup &G, hipStream_t st)
+int batch_launch_node(const BatchGroup &G, bool last, hipStream_t st)
 {
     if (G.kv == 1)
         hipLaunchKernelGGL((node_kernel_batch<P, R, 1>), dim3(G.nwg), dim3(256), 0, st,
@@ -1339,7 +1366,7 @@ int batch_launch_node(const BatchGroup &G, hipStream_t st)
         hipLaunchKernelGGL((node_kernel_batch<P, R, 0>), dim3(G.nwg), dim3(256), 0, st,
                            (const NodeArgs<R> *)G.d_nargs, (const int2 *)G.d_nown);
     HIPCHK(hipGetLastError());
-    if (G.rwg > 0) {
+    if (G.rwg > 0 && (last || !G.ride)) {
         hipLaunchKernelGGL((record_kernel_batch<P, R>), dim3(G.rwg), dim3(64), 0, st,
                            (const RecArgs<R> *)G.d_rargs + (size_t)G.phase * G.sims.size(),
                            (const int2 *)G.d_rown);
@@ -1348,13 +1375,13 @@ int batch_launch_node(const BatchGroup &G, hipStream_t st)
     return 0;
 }
 
-int batch_group_call(int what, BatchGroup &G, hipStream_t st)
+int batch_group_call(int what, BatchGroup &G, bool first, bool last, hipStream_t st)
 {
 #define S3D_BATCH_CASE(PP)                                                                  \
     case PP:                                                                                \
         if (what == 0) return G.fp32 ? batch_build_group<PP, float>(G) : batch_build_group<PP, double>(G); \
-        if (what == 1) return G.fp32 ? batch_launch_group<PP, float>(G, st) : batch_launch_group<PP, double>(G, st); \
-        return G.fp32 ? batch_launch_node<PP, float>(G, st) : batch_launch_node<PP, double>(G, st);
+        if (what == 1) return G.fp32 ? batch_launch_group<PP, float>(G, first, st) : batch_launch_group<PP, double>(G, first, st); \
+        return G.fp32 ? batch_launch_node<PP, float>(G, last, st) : batch_launch_node<PP, double>(G, last, st);
     switch (G.p) {
         S3D_BATCH_CASE(2)
         S3D_BATCH_CASE(3)
@@ -1385,9 +1412,10 @@ void batch_free_groups(s3d_batch *b)
     b->built = false;
 }
 
-// one batched iteration: every group's element kernel, then every group's
-// node and receiver kernels, then every counter advances
-int batch_launch_step(s3d_batch *b)
+// one batched iteration: every group's element kernel (with the receivers of
+// the iteration before), then every group's node kernel, and the receivers
+// after the last iteration of the call or of a captured chunk
+int batch_launch_step(s3d_batch *b, bool first, bool last)
 {
     // members with curl receivers: the strain parts of the start velocity,
     // before the element kernels change it
@@ -1399,13 +1427,10 @@ int batch_launch_step(s3d_batch *b)
         }
     for (auto &G : b->groups) {
         G.phase = b->phase;
-        if (int rc = batch_group_call(1, G, b->stream)) return rc;
+        if (int rc = batch_group_call(1, G, first, last, b->stream)) return rc;
     }
     for (auto &G : b->groups)
-        if (int rc = batch_group_call(2, G, b->stream)) return rc;
-    const int n = (int)b->sims.size();
-    hipLaunchKernelGGL(advance_many_kernel, dim3((n + 63) / 64), dim3(64), 0, b->stream, b->d_its, n);
-    HIPCHK(hipGetLastError());
+        if (int rc = batch_group_call(2, G, first, last, b->stream)) return rc;
     for (s3d_ctx *c : b->sims) advance_state(c);
     b->phase ^= 1;
     return 0;
@@ -1454,9 +1479,11 @@ int batch_build(s3d_batch *b)
             if (c->nel > big->nel) big = c;
         G.epb = big->epb;
         G.ll = big->fp32 ? kernel_variant(big) : 0;
+        G.ride = true;
+        for (const s3d_ctx *c : G.sims) G.ride = G.ride && (c->nrec_dev == 0 || receivers_ride(c));
     }
     for (auto &G : b->groups)
-        if (int rc = batch_group_call(0, G, b->stream)) return rc;
+        if (int rc = batch_group_call(0, G, false, false, b->stream)) return rc;
     b->built = true;
     return 0;
 }
@@ -2079,6 +2106,7 @@ int s3d_add_receiver(s3d_ctx *c, const int *exyz, const double *vm, int nch, con
         if (channels[q] < S3D_CH_VX || channels[q] > S3D_CH_FZ)
             return fail("unsupported receiver channel " + std::to_string(channels[q]));
     if (c->batches > 0) return refuse_batch_member(c, "add_receiver");
+    for (int q = 0; q < nch; ++q) c->rec_pressure |= channels[q] == S3D_CH_PRESSURE;
     c->rec_e.push_back((int)(ex + (long)c->g.nx * (ey + (long)c->g.ny * ez)));
     c->rec_nch.push_back(nch);
     c->rec_off.push_back((int)c->rec_ch.size());
@@ -2114,8 +2142,8 @@ int s3d_step(s3d_ctx *c, int nsteps)
             left -= GRAPH_CHUNK;
         }
     }
-    for (; left > 0; --left) {
-        int rc = launch_one(c);
+    for (bool first = true; left > 0; --left, first = false) {
+        int rc = launch_one(c, first, left == 1);
         if (rc) return rc;
         c->it += 1;
     }
@@ -2428,12 +2456,6 @@ int s3d_batch_create(int n, s3d_ctx *const *sims, s3d_batch **out)
     b->dev = sims[0]->dev;
     hipError_t e = hipStreamCreate(&b->stream);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&b->ev, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipMalloc(&b->d_its, sizeof(int *) * n);
-    if (e == hipSuccess) {
-        std::vector<int *> its(n);
-        for (int q = 0; q < n; ++q) its[q] = sims[q]->d_it;
-        e = hipMemcpy(b->d_its, its.data(), sizeof(int *) * n, hipMemcpyHostToDevice);
-    }
     if (e != hipSuccess) {
         if (b->stream) (void)hipStreamDestroy(b->stream);
         delete b;
@@ -2473,7 +2495,8 @@ int s3d_batch_step(s3d_batch *b, int nsteps)
             };
             HIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
             int rc = 0;
-            for (int q = 0; q < GRAPH_CHUNK && rc == 0; ++q) rc = batch_launch_step(b);
+            for (int q = 0; q < GRAPH_CHUNK && rc == 0; ++q)
+                rc = batch_launch_step(b, q == 0, q == GRAPH_CHUNK - 1);
             hipGraph_t g = nullptr;
             hipError_t e = hipStreamEndCapture(b->stream, &g);
             if (rc) {
@@ -2496,8 +2519,8 @@ int s3d_batch_step(s3d_batch *b, int nsteps)
             left -= GRAPH_CHUNK;
         }
     }
-    for (; left > 0; --left) {
-        if (int rc = batch_launch_step(b)) return rc;
+    for (bool first = true; left > 0; --left, first = false) {
+        if (int rc = batch_launch_step(b, first, left == 1)) return rc;
         for (s3d_ctx *c : b->sims) c->it += 1;
     }
     // and each member's stream after the batch
@@ -2520,7 +2543,6 @@ int s3d_batch_destroy(s3d_batch *b)
     (void)hipSetDevice(b->dev);
     (void)hipStreamSynchronize(b->stream);
     batch_free_groups(b);
-    dfree(b->d_its);
     if (b->ev) (void)hipEventDestroy(b->ev);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     for (s3d_ctx *c : b->sims) c->batches--;

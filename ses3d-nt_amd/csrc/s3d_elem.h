@@ -661,20 +661,170 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R> &a, int blk)
     }
 }
 
+// ---------------------------------------------------------------------------
+// receivers: one wave per receiver, all its channels
+// ---------------------------------------------------------------------------
+// The curl formulas (src/config/channel_mod.f90:620-774 for receivers,
+// src/volume_snapshot.f90:238-245 for snapshots) from the parts of a step's
+// start velocity and the velocity vx, vy at its end; comp 0, 1, 2 =
+// rot_vx, rot_vy, rot_vz.
+__device__ inline double curl_formula(int comp, const double part[6], double vxn, double vyn, double r,
+                                      double rs, double ct, double st)
+{
+    if (comp == 0) return -vyn / r + part[0] / rs + part[3];
+    if (comp == 1) return -part[4] + (vxn - part[1]) / r;
+    return (part[2] + vyn * ct - part[5] / st) / r;
+}
+
+template <typename R>
+struct RecArgs {
+    int n;      // receivers
+    int pressure;   // some of them record the pressure (the only use of sig)
+    int nx, ny, nel, nt;
+    int ns;     // components of the state block
+    gptr<const R> vx, vy, vz, lx, ly, lz, sig;
+    gptr<const bf16> hx, hy, hz;  // BF16 velocity compensation (lx.. null) or null
+    gptr<const int> rec_rot;      // curl slot per receiver, -1 none (null: no curl receivers)
+    gptr<const double> rot_buf;   // per curl slot [10][NP], see curl_strain_kernel
+    gptr<const int> rec_e, rec_nch, rec_off, rec_ch;  // channels of receiver r: rec_ch[rec_off[r] + q]
+    gptr<const double> rec_vm;
+    gptr<double> traces;          // [sum of channels][nt], receiver r's at rec_off[r]
+    gptr<const int> it_dev;
+    // sources, for the echo channels: slot per element (null: no sources),
+    // channel row per slot and component, coefficients, source-time table
+    gptr<const int> src_slot, src_chan;
+    gptr<const double> src_coef, stf;
+};
+
+// Receiver r's samples of the iteration just completed, *it_dev (the node
+// kernel has advanced the counter), by the 64 lanes of one wave. CURL: the
+// receiver may have curl channels.
+template <int P, typename R, bool CURL>
+__device__ __forceinline__ void record_body(const RecArgs<R> &a, int r)
+{
+    constexpr int P1 = P + 1, NP = P1 * P1 * P1;
+    const int it = *a.it_dev;
+    if (it < 1 || it > a.nt) return;
+    const int lane = threadIdx.x & 63;
+    const int e = a.rec_e[r];
+    const int ex = e % a.nx, ey = (e / a.nx) % a.ny, ez = e / (a.nx * a.ny);
+    double acc[CURL ? 7 : 4] = {};   // vx, vy, vz, pressure, rot_vx, rot_vy, rot_vz
+    const int rs = CURL && a.rec_rot ? a.rec_rot[r] : -1;
+    for (int n = lane; n < NP; n += 64) {
+        const int i = n % P1, j = (n / P1) % P1, k = n / (P1 * P1);
+        const long u = unique_index<P>(ex, ey, ez, i, j, k, a.nx, a.ny);
+        const double w = a.rec_vm[(long)r * NP + n];
+        // compensated velocity: value = hi - lo
+        const double vxn = (double)a.vx[u] - vel_lo(a.lx, a.hx, u);
+        const double vyn = (double)a.vy[u] - vel_lo(a.ly, a.hy, u);
+        acc[0] += w * vxn;
+        acc[1] += w * vyn;
+        acc[2] += w * ((double)a.vz[u] - vel_lo(a.lz, a.hz, u));
+        if (a.pressure) {
+            const double tr = (double)a.sig[em_index(e, a.ns, XX, NP, n)] + (double)a.sig[em_index(e, a.ns, YY, NP, n)] +
+                              (double)a.sig[em_index(e, a.ns, ZZ, NP, n)];
+            acc[3] += -((double)(1.0f / 3.0f) * tr) * w;
+        }
+        if constexpr (CURL) {
+            if (rs >= 0) {
+                // curl channels (src/config/channel_mod.f90:620-774): strain-rate
+                // parts of the step's start velocity, this velocity at its end
+                const double *b = a.rot_buf + (long)rs * 10 * NP + n;
+                double part[6];
+#pragma unroll
+                for (int c = 0; c < 6; ++c) part[c] = b[c * NP];
+                const double rr = b[6 * NP], rst = b[7 * NP], ct = b[8 * NP], st = b[9 * NP];
+#pragma unroll
+                for (int c = 0; c < 3; ++c) acc[4 + c] += w * curl_formula(c, part, vxn, vyn, rr, rst, ct, st);
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < (CURL ? 7 : 4); ++c)
+        for (int off = 32; off > 0; off >>= 1) acc[c] += __shfl_down(acc[c], off, 64);
+    // source-echo channels: add(it) of this step wrote, per component c with
+    // a source in this element, src_c = -stf(it) * coef_c (an assignment: the
+    // last source of the element wins, as in add_m** / add_f*,
+    // src/config/channel_mod.f90:859-1095); record_m** / record_f* sum vm *
+    // src_c (:871-1085). mxx .. mzz, fx, fy, fz; zero in other elements.
+    const int slot = a.src_slot ? a.src_slot[e] : -1;
+    auto echo = [&](int c) {
+        double s = 0.0;
+        const int ch = slot >= 0 ? a.src_chan[slot * 9 + c] : -1;
+        if (ch < 0) return s;
+        const double sd = a.stf[(long)ch * a.nt + (it - 1)];
+        if (sd != 0.0)
+            for (int n = lane; n < NP; n += 64)
+                s += a.rec_vm[(long)r * NP + n] * -(sd * a.src_coef[((long)slot * 9 + c) * NP + n]);
+        for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+        return s;
+    };
+    const int nch = a.rec_nch[r];
+    const int off = a.rec_off[r];
+    for (int q = 0; q < nch; ++q) {
+        const int ch = a.rec_ch[off + q];
+        double val = 0.0;
+        switch (ch) {
+        case 0: val = acc[0]; break;          // vx
+        case 1: val = acc[1]; break;          // vy
+        case 2: val = acc[2]; break;          // vz
+        case 3: val = -acc[0]; break;         // n = -vx
+        case 4: val = acc[1]; break;          // e = vy
+        case 5: val = acc[2]; break;          // z = vz
+        case 6: val = acc[3]; break;          // pressure
+        case 7: if constexpr (CURL) val = acc[4]; break;   // rot_vx
+        case 8: if constexpr (CURL) val = acc[5]; break;   // rot_vy
+        case 9: if constexpr (CURL) val = acc[6]; break;   // rot_vz
+        default:                              // mxx .. mzz, fx, fy, fz
+            if (ch >= 10 && ch < 19) val = echo(ch - 10);
+            break;
+        }
+        if (lane == 0) a.traces[((long)off + q) * a.nt + (it - 1)] = val;
+    }
+}
+
+// Workgroups of an element launch that record the receivers of the iteration
+// before it, one receiver per wave, ahead of the tiles: rounded up to a
+// multiple of 8 so that the tiles' order on the XCDs stays. A receiver launch
+// of its own takes 7 to 8 us of a 25 us step at 12x12x8, 13 to 20 us with 32
+// to 256 receivers, almost all of it latency that the tiles hide here: with
+// the step counter advanced by the node kernel a step at 12x12x8, order 4, FP64
+// in captured chunks goes from 24.6 to 15.6 us.
+__host__ __device__ inline int record_blocks(int receivers, int lanes)
+{
+    const int per = lanes / 64;
+    return ((receivers + per - 1) / per + 7) / 8 * 8;
+}
+
 template <int P, int E, typename R, int VM, bool S16, int KS, int LL>
 __global__ void __launch_bounds__((Shape<P, E>::NT))
-elem_kernel(const ElemArgs<R> a)
+elem_kernel(const ElemArgs<R> a, const RecArgs<R> rec)
 {
-    elem_body<P, E, R, VM, S16, KS, LL>(a, chunk_block(blockIdx.x, gridDim.x, a.remap));
+    constexpr int NT = Shape<P, E>::NT;
+    const int nb = record_blocks(rec.n, NT), b = (int)blockIdx.x - nb;
+    if (b < 0) {
+        const int r = (int)blockIdx.x * (NT / 64) + (int)(threadIdx.x >> 6);
+        if (r < rec.n) record_body<P, R, false>(rec, r);
+        return;
+    }
+    elem_body<P, E, R, VM, S16, KS, LL>(a, chunk_block(b, gridDim.x - nb, a.remap));
 }
 
 template <int P, int E, typename R, int VM, int KS, int LL>
 __global__ void __launch_bounds__((Shape<P, E>::NT))
-elem_kernel_batch(const ElemArgs<R> *__restrict__ args, const int2 *__restrict__ own)
+elem_kernel_batch(const ElemArgs<R> *__restrict__ args, const int2 *__restrict__ own,
+                  const RecArgs<R> *__restrict__ recs, const int2 *__restrict__ rown, int nrec)
 {
+    constexpr int NT = Shape<P, E>::NT;
+    const int nb = record_blocks(nrec, NT), b = (int)blockIdx.x - nb;
+    if (b < 0) {
+        const int r = (int)blockIdx.x * (NT / 64) + (int)(threadIdx.x >> 6);
+        if (r < nrec) record_body<P, R, false>(recs[rown[r].x], rown[r].y);
+        return;
+    }
     // (simulation, its workgroup index), in XCD-aware order over the whole
     // batch
-    const int2 o = own[chunk_block(blockIdx.x, gridDim.x, 1)];
+    const int2 o = own[chunk_block(b, gridDim.x - nb, 1)];
     elem_body<P, E, R, VM, false, KS, LL>(args[o.x], o.y);
 }
 

@@ -22,47 +22,47 @@ unsigned tiles(long nel) { return (unsigned)((nel + Shape<P, E>::EPB - 1) / Shap
 
 // stress compensation (FP32 only)
 template <int P, int E, typename R, int VM, bool S16, int LL>
-void launch_ks(int ks, const ElemArgs<R> &ea, hipStream_t st, unsigned ge)
+void launch_ks(int ks, const ElemArgs<R> &ea, const RecArgs<R> &ra, hipStream_t st, unsigned ge)
 {
     constexpr int NT = Shape<P, E>::NT;
     if (ks == 1)
-        hipLaunchKernelGGL((elem_kernel<P, E, R, VM, S16, 1, LL>), dim3(ge), dim3(NT), 0, st, ea);
+        hipLaunchKernelGGL((elem_kernel<P, E, R, VM, S16, 1, LL>), dim3(ge), dim3(NT), 0, st, ea, ra);
     else if (ks == 2)
-        hipLaunchKernelGGL((elem_kernel<P, E, R, VM, S16, 2, LL>), dim3(ge), dim3(NT), 0, st, ea);
+        hipLaunchKernelGGL((elem_kernel<P, E, R, VM, S16, 2, LL>), dim3(ge), dim3(NT), 0, st, ea, ra);
     else
-        hipLaunchKernelGGL((elem_kernel<P, E, R, VM, S16, 0, LL>), dim3(ge), dim3(NT), 0, st, ea);
+        hipLaunchKernelGGL((elem_kernel<P, E, R, VM, S16, 0, LL>), dim3(ge), dim3(NT), 0, st, ea, ra);
 }
 
 // kernel variant and stress compensation: FP32 only; FP64 and the
 // BF16-static kernels use variant 0 without compensation words
 template <int P, int E, typename R, int VM, bool S16>
-void launch_ll(int ks, int ll, const ElemArgs<R> &ea, hipStream_t st, unsigned ge)
+void launch_ll(int ks, int ll, const ElemArgs<R> &ea, const RecArgs<R> &ra, hipStream_t st, unsigned ge)
 {
     if constexpr (std::is_same<R, float>::value) {
         if constexpr (!S16) {
-            if (ll == 1) return launch_ks<P, E, R, VM, S16, 1>(ks, ea, st, ge);
-            if (ll == 2) return launch_ks<P, E, R, VM, S16, 2>(ks, ea, st, ge);
+            if (ll == 1) return launch_ks<P, E, R, VM, S16, 1>(ks, ea, ra, st, ge);
+            if (ll == 2) return launch_ks<P, E, R, VM, S16, 2>(ks, ea, ra, st, ge);
         }
-        launch_ks<P, E, R, VM, S16, 0>(ks, ea, st, ge);
+        launch_ks<P, E, R, VM, S16, 0>(ks, ea, ra, st, ge);
     } else {
-        hipLaunchKernelGGL((elem_kernel<P, E, R, VM, S16, 0, 0>), dim3(ge), dim3(Shape<P, E>::NT), 0, st, ea);
+        hipLaunchKernelGGL((elem_kernel<P, E, R, VM, S16, 0, 0>), dim3(ge), dim3(Shape<P, E>::NT), 0, st, ea, ra);
     }
 }
 
 template <int P, int E, typename R>
-void launch_vm(const ElemLaunch &l, const ElemArgs<R> &ea, hipStream_t st)
+void launch_vm(const ElemLaunch &l, const ElemArgs<R> &ea, const RecArgs<R> &ra, hipStream_t st)
 {
-    const unsigned ge = tiles<P, E>(l.nel);
+    const unsigned ge = tiles<P, E>(l.nel) + record_blocks(ra.n, Shape<P, E>::NT);
     if constexpr (std::is_same<R, float>::value && E == 0) {
         if (l.bf16_static) {
-            if (l.vm == 6) return launch_ll<P, 0, float, 6, true>(l.ks, 0, ea, st, ge);
-            if (l.vm == 5) return launch_ll<P, 0, float, 5, true>(l.ks, 0, ea, st, ge);
-            return launch_ll<P, 0, float, 0, true>(l.ks, 0, ea, st, ge);
+            if (l.vm == 6) return launch_ll<P, 0, float, 6, true>(l.ks, 0, ea, ra, st, ge);
+            if (l.vm == 5) return launch_ll<P, 0, float, 5, true>(l.ks, 0, ea, ra, st, ge);
+            return launch_ll<P, 0, float, 0, true>(l.ks, 0, ea, ra, st, ge);
         }
     }
-    if (l.vm == 6) return launch_ll<P, E, R, 6, false>(l.ks, l.ll, ea, st, ge);
-    if (l.vm == 5) return launch_ll<P, E, R, 5, false>(l.ks, l.ll, ea, st, ge);
-    launch_ll<P, E, R, 0, false>(l.ks, l.ll, ea, st, ge);
+    if (l.vm == 6) return launch_ll<P, E, R, 6, false>(l.ks, l.ll, ea, ra, st, ge);
+    if (l.vm == 5) return launch_ll<P, E, R, 5, false>(l.ks, l.ll, ea, ra, st, ge);
+    launch_ll<P, E, R, 0, false>(l.ks, l.ll, ea, ra, st, ge);
 }
 
 template <int P, int E, typename R, int VM, int KS>
@@ -70,17 +70,22 @@ void batch_ll(const ElemBatchLaunch &l, hipStream_t st)
 {
     constexpr int NT = Shape<P, E>::NT;
     const ElemArgs<R> *args = (const ElemArgs<R> *)l.args;
+    const RecArgs<R> *recs = (const RecArgs<R> *)l.recs;
+    const unsigned nwg = l.nwg + record_blocks(l.nrec, NT);
     if constexpr (std::is_same<R, float>::value) {
         if (l.ll == 1) {
-            hipLaunchKernelGGL((elem_kernel_batch<P, E, R, VM, KS, 1>), dim3(l.nwg), dim3(NT), 0, st, args, l.own);
+            hipLaunchKernelGGL((elem_kernel_batch<P, E, R, VM, KS, 1>), dim3(nwg), dim3(NT), 0, st, args, l.own, recs,
+                               l.rown, l.nrec);
             return;
         }
         if (l.ll == 2) {
-            hipLaunchKernelGGL((elem_kernel_batch<P, E, R, VM, KS, 2>), dim3(l.nwg), dim3(NT), 0, st, args, l.own);
+            hipLaunchKernelGGL((elem_kernel_batch<P, E, R, VM, KS, 2>), dim3(nwg), dim3(NT), 0, st, args, l.own, recs,
+                               l.rown, l.nrec);
             return;
         }
     }
-    hipLaunchKernelGGL((elem_kernel_batch<P, E, R, VM, KS, 0>), dim3(l.nwg), dim3(NT), 0, st, args, l.own);
+    hipLaunchKernelGGL((elem_kernel_batch<P, E, R, VM, KS, 0>), dim3(nwg), dim3(NT), 0, st, args, l.own, recs,
+                               l.rown, l.nrec);
 }
 
 template <int P, int E, typename R, int VM>
@@ -107,17 +112,17 @@ void batch_vm(const ElemBatchLaunch &l, hipStream_t st)
 // lanes, besides the default. The BF16-static kernel exists for the
 // default tile only.
 template <int P, typename R>
-hipError_t launch_elem_kernel(const ElemLaunch &l, const ElemArgs<R> &ea, hipStream_t st)
+hipError_t launch_elem_kernel(const ElemLaunch &l, const ElemArgs<R> &ea, const RecArgs<R> &ra, hipStream_t st)
 {
     const int epb = (std::is_same<R, float>::value && l.bf16_static) ? 0 : l.epb;
     bool done = false;
     if constexpr (extra_tile<P, 1>())
-        if (epb == 1) { launch_vm<P, 1, R>(l, ea, st); done = true; }
+        if (epb == 1) { launch_vm<P, 1, R>(l, ea, ra, st); done = true; }
     if constexpr (extra_tile<P, 2>())
-        if (epb == 2) { launch_vm<P, 2, R>(l, ea, st); done = true; }
+        if (epb == 2) { launch_vm<P, 2, R>(l, ea, ra, st); done = true; }
     if constexpr (extra_tile<P, 4>())
-        if (epb == 4) { launch_vm<P, 4, R>(l, ea, st); done = true; }
-    if (!done) launch_vm<P, 0, R>(l, ea, st);
+        if (epb == 4) { launch_vm<P, 4, R>(l, ea, ra, st); done = true; }
+    if (!done) launch_vm<P, 0, R>(l, ea, ra, st);
     return hipGetLastError();
 }
 
@@ -139,8 +144,8 @@ hipError_t launch_elem_batch(const ElemBatchLaunch &l, hipStream_t st)
     return hipGetLastError();
 }
 
-template hipError_t launch_elem_kernel<S3D_ELEM_P, float>(const ElemLaunch &, const ElemArgs<float> &, hipStream_t);
-template hipError_t launch_elem_kernel<S3D_ELEM_P, double>(const ElemLaunch &, const ElemArgs<double> &, hipStream_t);
+template hipError_t launch_elem_kernel<S3D_ELEM_P, float>(const ElemLaunch &, const ElemArgs<float> &, const RecArgs<float> &, hipStream_t);
+template hipError_t launch_elem_kernel<S3D_ELEM_P, double>(const ElemLaunch &, const ElemArgs<double> &, const RecArgs<double> &, hipStream_t);
 template hipError_t launch_elem_batch<S3D_ELEM_P, float>(const ElemBatchLaunch &, hipStream_t);
 template hipError_t launch_elem_batch<S3D_ELEM_P, double>(const ElemBatchLaunch &, hipStream_t);
 

@@ -157,6 +157,7 @@ struct NodeArgs {
     gptr<const double> px, py, pz;
     double alpha;
     int taper_on;
+    gptr<int> it_dev;          // iterations completed, advanced by the first lane
 };
 
 // Compensation term of a compensated velocity component at unique node u,

@@ -1,7 +1,7 @@
 // s3d_kernels.hip -- gfx950 kernels of the forward time step.
 //
 // One time step (reference src/ses3d-nt.F90:240-270 around
-// src/evolution.f90:87-444) is two kernels plus a tiny receiver kernel:
+// src/evolution.f90:87-444) is two kernels:
 //
 //   elem_kernel  one workgroup per EPB elements, one lane per element-local
 //                node. Gathers the element's velocity into LDS, forms the
@@ -15,7 +15,10 @@
 //                (K10, src/communicate_fields.F90:48-79; deterministic, no
 //                atomics), multiplies by 1/M (K9), integrates the velocity
 //                (K12, optional compensated summation) and tapers it (K13).
-//   record_kernel one wave per receiver: sum vm * field over the element.
+//                Its first lane advances the step counter.
+// and the receivers (one wave each: sum vm * field over the element), which
+// ride in the next step's element kernel, or in record_kernel after the last
+// step of a call.
 //
 // HBM bytes per element-local node and step (FP32, Kahan on v, visco):
 //   stress 24 r + 24 w, memory variables 72 r + 72 w (60 + 60 in the
@@ -39,6 +42,10 @@ __device__ __forceinline__ void node_body(const NodeArgs<R> &a, long tid)
     constexpr int P1 = P + 1, PB = P * P * P;
     constexpr int NL = P1 * P1, NM = NL * P;   // force layout, see force_index
     if (tid >= a.nblk * PB) return;
+    // the iteration is complete with this kernel: advance the step counter
+    // (the element kernel has read it, the receivers read it afterwards). A
+    // launch of its own for this took 4.5 us per step of a captured chunk.
+    if (tid == 0) a.it_dev[0] = a.it_dev[0] + 1;
     // 32-bit index arithmetic (s3d_create keeps unique nodes below 2^32 and
     // elements below 2^31): 64-bit divisions by the run-time block counts
     // took about 40 % of the kernel's VALU instructions
@@ -144,127 +151,6 @@ node_kernel_batch(const NodeArgs<R> *__restrict__ args, const int2 *__restrict__
 {
     const int2 o = own[blockIdx.x];
     node_body<P, R, KV>(args[o.x], (long)o.y * blockDim.x + threadIdx.x);
-}
-
-// ---------------------------------------------------------------------------
-// receivers: one wave per receiver, all its channels
-// ---------------------------------------------------------------------------
-// The curl formulas (src/config/channel_mod.f90:620-774 for receivers,
-// src/volume_snapshot.f90:238-245 for snapshots) from the parts of a step's
-// start velocity and the velocity vx, vy at its end; comp 0, 1, 2 =
-// rot_vx, rot_vy, rot_vz.
-__device__ inline double curl_formula(int comp, const double part[6], double vxn, double vyn, double r,
-                                      double rs, double ct, double st)
-{
-    if (comp == 0) return -vyn / r + part[0] / rs + part[3];
-    if (comp == 1) return -part[4] + (vxn - part[1]) / r;
-    return (part[2] + vyn * ct - part[5] / st) / r;
-}
-
-template <typename R>
-struct RecArgs {
-    int nx, ny, nel, nt;
-    int ns;     // components of the state block
-    gptr<const R> vx, vy, vz, lx, ly, lz, sig;
-    gptr<const bf16> hx, hy, hz;  // BF16 velocity compensation (lx.. null) or null
-    gptr<const int> rec_rot;      // curl slot per receiver, -1 none (null: no curl receivers)
-    gptr<const double> rot_buf;   // per curl slot [10][NP], see curl_strain_kernel
-    gptr<const int> rec_e, rec_nch, rec_off, rec_ch;  // channels of receiver r: rec_ch[rec_off[r] + q]
-    gptr<const double> rec_vm;
-    gptr<double> traces;          // [sum of channels][nt], receiver r's at rec_off[r]
-    gptr<const int> it_dev;
-    // sources, for the echo channels: slot per element (null: no sources),
-    // channel row per slot and component, coefficients, source-time table
-    gptr<const int> src_slot, src_chan;
-    gptr<const double> src_coef, stf;
-};
-
-template <int P, typename R>
-__device__ __forceinline__ void record_body(const RecArgs<R> &a, int r)
-{
-    constexpr int P1 = P + 1, NP = P1 * P1 * P1;
-    // records iteration it = *it_dev + 1 (the counter advances after this kernel)
-    const int it = *a.it_dev + 1;
-    if (it < 1 || it > a.nt) return;
-    const int lane = threadIdx.x;
-    const int e = a.rec_e[r];
-    const int ex = e % a.nx, ey = (e / a.nx) % a.ny, ez = e / (a.nx * a.ny);
-    // source-echo channels: add(it) of this step wrote, per component c with
-    // a source in this element, src_c = -stf(it) * coef_c (an assignment: the
-    // last source of the element wins, as in add_m** / add_f*,
-    // src/config/channel_mod.f90:859-1095); record_m** / record_f* sum vm *
-    // src_c (:871-1085)
-    const int slot = a.src_slot ? a.src_slot[e] : -1;
-    double sd[9];
-#pragma unroll
-    for (int c = 0; c < 9; ++c) {
-        const int ch = slot >= 0 ? a.src_chan[slot * 9 + c] : -1;
-        sd[c] = ch >= 0 ? a.stf[(long)ch * a.nt + (it - 1)] : 0.0;
-    }
-    double acc[7] = {0, 0, 0, 0, 0, 0, 0};   // vx, vy, vz, pressure, rot_vx, rot_vy, rot_vz
-    double accs[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};   // mxx .. mzz, fx, fy, fz
-    const int rs = a.rec_rot ? a.rec_rot[r] : -1;
-    for (int n = lane; n < NP; n += 64) {
-        const int i = n % P1, j = (n / P1) % P1, k = n / (P1 * P1);
-        const long u = unique_index<P>(ex, ey, ez, i, j, k, a.nx, a.ny);
-        const double w = a.rec_vm[(long)r * NP + n];
-        // compensated velocity: value = hi - lo
-        const double vxn = (double)a.vx[u] - vel_lo(a.lx, a.hx, u);
-        const double vyn = (double)a.vy[u] - vel_lo(a.ly, a.hy, u);
-        acc[0] += w * vxn;
-        acc[1] += w * vyn;
-        acc[2] += w * ((double)a.vz[u] - vel_lo(a.lz, a.hz, u));
-        const double tr = (double)a.sig[em_index(e, a.ns, XX, NP, n)] + (double)a.sig[em_index(e, a.ns, YY, NP, n)] +
-                          (double)a.sig[em_index(e, a.ns, ZZ, NP, n)];
-        acc[3] += -((double)(1.0f / 3.0f) * tr) * w;
-        if (rs >= 0) {
-            // curl channels (src/config/channel_mod.f90:620-774): strain-rate
-            // parts of the step's start velocity, this velocity at its end
-            const double *b = a.rot_buf + (long)rs * 10 * NP + n;
-            double part[6];
-#pragma unroll
-            for (int c = 0; c < 6; ++c) part[c] = b[c * NP];
-            const double rr = b[6 * NP], rst = b[7 * NP], ct = b[8 * NP], st = b[9 * NP];
-#pragma unroll
-            for (int c = 0; c < 3; ++c) acc[4 + c] += w * curl_formula(c, part, vxn, vyn, rr, rst, ct, st);
-        }
-        if (slot >= 0) {
-#pragma unroll
-            for (int c = 0; c < 9; ++c)
-                if (sd[c] != 0.0)
-                    accs[c] += w * -(sd[c] * a.src_coef[((long)slot * 9 + c) * NP + n]);
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < 7; ++c)
-        for (int off = 32; off > 0; off >>= 1) acc[c] += __shfl_down(acc[c], off, 64);
-#pragma unroll
-    for (int c = 0; c < 9; ++c)
-        for (int off = 32; off > 0; off >>= 1) accs[c] += __shfl_down(accs[c], off, 64);
-    if (lane == 0) {
-        const int nch = a.rec_nch[r];
-        const int off = a.rec_off[r];
-        for (int q = 0; q < nch; ++q) {
-            const int ch = a.rec_ch[off + q];
-            double val = 0.0;
-            switch (ch) {
-            case 0: val = acc[0]; break;          // vx
-            case 1: val = acc[1]; break;          // vy
-            case 2: val = acc[2]; break;          // vz
-            case 3: val = -acc[0]; break;         // n = -vx
-            case 4: val = acc[1]; break;          // e = vy
-            case 5: val = acc[2]; break;          // z = vz
-            case 6: val = acc[3]; break;          // pressure
-            case 7: val = acc[4]; break;          // rot_vx
-            case 8: val = acc[5]; break;          // rot_vy
-            case 9: val = acc[6]; break;          // rot_vz
-            default:                              // mxx .. mzz, fx, fy, fz
-                if (ch >= 10 && ch < 19) val = accs[ch - 10];
-                break;
-            }
-            a.traces[((long)off + q) * a.nt + (it - 1)] = val;
-        }
-    }
 }
 
 // Strain-rate parts of the curl receiver channels (reference record_rot_v*,
@@ -404,31 +290,20 @@ struct CurlSrc {
     }
 };
 
+// The receivers' own launch: after the last step of a call, and after every
+// step where the element kernel of the next one cannot record (curl channels,
+// or a stress block updated in place).
 template <int P, typename R>
 __global__ void __launch_bounds__(64) record_kernel(const RecArgs<R> a)
 {
-    record_body<P, R>(a, blockIdx.x);
+    record_body<P, R, true>(a, blockIdx.x);
 }
 
 template <int P, typename R>
 __global__ void __launch_bounds__(64) record_kernel_batch(const RecArgs<R> *__restrict__ args, const int2 *__restrict__ own)
 {
     const int2 o = own[blockIdx.x];
-    record_body<P, R>(args[o.x], o.y);
-}
-
-// End of one iteration: advance the device step counter. A single lane
-// stores through the vector path.
-__global__ void __launch_bounds__(64) advance_kernel(int *it_dev)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) it_dev[0] = it_dev[0] + 1;
-}
-
-// End of one batched iteration: advance every simulation's counter.
-__global__ void __launch_bounds__(64) advance_many_kernel(int *const *its, int n)
-{
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < n) its[s][0] = its[s][0] + 1;
+    record_body<P, R, true>(args[o.x], o.y);
 }
 
 // ---------------------------------------------------------------------------

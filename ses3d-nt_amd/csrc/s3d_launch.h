@@ -31,14 +31,20 @@ struct ElemLaunch {
 // phase (device memory) and its workgroup -> (member, member's workgroup) map.
 struct ElemBatchLaunch {
     int vm, ks, ll, epb;   // as in ElemLaunch, shared by the group's members
-    unsigned nwg;          // workgroups of the launch
+    unsigned nwg;          // element workgroups of the launch
     const void *args;      // ElemArgs<R>[members]
     const int2 *own;       // [nwg]
+    // receivers of the step before (0: none): RecArgs<R>[members], (member,
+    // its receiver) per receiver
+    int nrec;
+    const void *recs;
+    const int2 *rown;
 };
 
-// Both return the launch status (hipGetLastError after the launch).
+// Both return the launch status (hipGetLastError after the launch). ra: the
+// receivers that the launch records for the step before (ra.n = 0: none).
 template <int P, typename R>
-hipError_t launch_elem_kernel(const ElemLaunch &l, const ElemArgs<R> &ea, hipStream_t st);
+hipError_t launch_elem_kernel(const ElemLaunch &l, const ElemArgs<R> &ea, const RecArgs<R> &ra, hipStream_t st);
 
 template <int P, typename R>
 hipError_t launch_elem_batch(const ElemBatchLaunch &l, hipStream_t st);
