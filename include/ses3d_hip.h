@@ -141,7 +141,7 @@ int s3d_destroy(s3d_ctx *ctx);
  * receivers and step counter; it is ready to step (no s3d_init). The model's
  * simulation must outlive it. No counterpart in the reference, which
  * superposes several sources in one wavefield; this is the batch axis of
- * many sources sharing one Earth model (batched source-innermost by
+ * many sources sharing one Earth model (batched by
  * s3d_batch_create). */
 int s3d_create_shared(s3d_ctx *model, s3d_ctx **out);
 
@@ -340,10 +340,7 @@ int s3d_device_bytes(s3d_ctx *ctx, double *bytes);
  * counterpart in the reference, which runs one event per process group;
  * this is the batch axis of the workloads with many independent regional
  * simulations. A member may not be stepped on its own while its batch steps.
- * When every member of a group shares one model (s3d_create_shared), the
- * group's workgroups run source-innermost: all members' workgroups of one
- * element tile follow each other, and the shared static fields are read
- * from HBM once per tile. */
+ * Members may share one model (s3d_create_shared). */
 typedef struct s3d_batch s3d_batch;
 int s3d_batch_create(int n, s3d_ctx *const *sims, s3d_batch **out);
 int s3d_batch_step(s3d_batch *batch, int nsteps);

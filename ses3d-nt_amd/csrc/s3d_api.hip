@@ -1283,27 +1283,19 @@ int batch_build_group_e(BatchGroup &G)
     G.ewg = es[n];
     G.nwg = ns[n];
     G.rwg = rs[n];
-    // Simulations that share one model (s3d_create_shared) run
-    // source-innermost: the workgroups of one element tile (or node range)
-    // for every member follow each other, so the shared moduli, tau and dt/M
-    // come from HBM once per tile and from cache for the other members.
-    bool interleave = n > 1;
-    for (int q = 1; q < n && interleave; ++q) interleave = model_of(G.sims[q]) == model_of(G.sims[0]);
-    auto owners = [n](const std::vector<int> &st, bool inter) {
+    // The workgroups of one member follow each other, also where the members
+    // share one model (s3d_create_shared). The other order there, all
+    // members' workgroups of one tile together so that the shared moduli come
+    // from HBM once, walks as many state blocks at a time as there are
+    // members: 6 sources on 40x40x20 elements 1264 us a step against 1228, on
+    // 96x96x32 11.85 ms against 11.02, 4 on 128x128x48 20.9 against 20.7.
+    auto owners = [n](const std::vector<int> &st) {
         std::vector<int2> o(st[n]);
-        if (inter) {
-            const int per = st[1] - st[0];   // members share the mesh and tile
-            for (int w = 0; w < per; ++w)
-                for (int q = 0; q < n; ++q) o[(size_t)w * n + q] = make_int2(q, w);
-        } else {
-            for (int q = 0; q < n; ++q)
-                for (int w = st[q]; w < st[q + 1]; ++w) o[w] = make_int2(q, w - st[q]);
-        }
+        for (int q = 0; q < n; ++q)
+            for (int w = st[q]; w < st[q + 1]; ++w) o[w] = make_int2(q, w - st[q]);
         return o;
     };
-    // receivers differ between members: their launch stays member-major
-    const std::vector<int2> eo = owners(es, interleave), no = owners(ns, interleave),
-                            ro = owners(rs, false);
+    const std::vector<int2> eo = owners(es), no = owners(ns), ro = owners(rs);
     HIPCHK(hipMalloc(&G.d_eargs, sizeof(ElemArgs<R>) * 2 * n));
     HIPCHK(hipMalloc(&G.d_nargs, sizeof(NodeArgs<R>) * n));
     HIPCHK(hipMalloc(&G.d_rargs, sizeof(RecArgs<R>) * 2 * n));
