@@ -759,27 +759,31 @@ struct CflRun {
 };
 
 // ---- fields to and from the host ----
-// A field crosses in chunks of at most IO_BYTES: export_field / import_field
-// work on a chunk in pinned host memory, and host threads copy between it and
-// the caller's array, each with a pinned buffer and an event of its own, so
-// that the copies of some chunks (and the first touch of the caller's pages)
-// run while the host link carries others: a velocity component at 96x96x48,
-// order 4 (442 MB into fresh pages) takes 45 ms on one thread, 16.8 ms on 4,
-// 13.4 ms on 8 and 16 threads (into touched pages 9.4 ms, 47 GB/s); chunks of
-// 2 MB 14.2 ms, 1 MB 16.5 ms. 32 MB: 1.29 ms on 4 threads, 1.48 ms on 8, so
-// the threads grow with the chunks. (One hipMemcpy from a device buffer:
-// 44 ms, and 254 ms for a stress component whose compensation the host
-// subtracted.) Buffers are taken from a process-wide list for the duration of
-// one call, at most IO_KEPT sets per device stay on it, and the last
-// simulation of a device frees them.
+// A field crosses in chunks of IO_LEAST to IO_BYTES (an eighth of it in
+// between): export_field / import_field work on a chunk in pinned host memory,
+// and host threads copy between it and the caller's array, each with two
+// pinned buffers, so that the copies of some chunks (and the first touch of
+// the caller's pages) run while the host link carries others. Reading, one
+// thread per IO_PER_THREAD chunks: 442 MB into fresh pages (a velocity
+// component at 96x96x48, order 4) take 35 ms on one thread, 14.9 ms on 4,
+// 12.3 ms on 8; 32 MB 2.6 ms on one, 1.8 ms on 3; in 2 MB chunks the 442 MB
+// take 13.5 ms, in 1 MB chunks 15.8 ms, but a 4 MB field 0.7 ms in place of
+// 0.8 ms. (One hipMemcpy from a device buffer: 44 ms, and 254 ms for a stress
+// component whose compensation the host subtracted.) Writing, two threads
+// reach what the link takes, 9.2 ms for the 442 MB (hipMemcpy: 16.4 ms), and
+// more only get in the way of a caller whose own threads still spin. Buffers
+// are taken from a process-wide list for the duration of one call, at most
+// IO_KEPT sets per device stay on it, and the last simulation of a device
+// frees them.
 constexpr int IO_THREADS = 8;
-constexpr size_t IO_BYTES = 4u << 20;
+constexpr size_t IO_BYTES = 4u << 20, IO_LEAST = 1u << 20;
+constexpr long IO_PER_THREAD = 4;
 constexpr size_t IO_KEPT = 2;
 
 struct IoBuffers {
     int dev = 0;
-    char *buf[IO_THREADS] = {};
-    hipEvent_t ev[IO_THREADS] = {};
+    char *buf[2 * IO_THREADS] = {};
+    hipEvent_t ev[2 * IO_THREADS] = {};
 };
 
 std::mutex g_io_mutex;
@@ -788,7 +792,7 @@ int g_live[MAX_DEVICES] = {};   // simulations per device
 
 void io_delete(IoBuffers *b)
 {
-    for (int t = 0; t < IO_THREADS; ++t) {
+    for (int t = 0; t < 2 * IO_THREADS; ++t) {
         if (b->ev[t]) (void)hipEventDestroy(b->ev[t]);
         if (b->buf[t]) (void)hipHostFree(b->buf[t]);
     }
@@ -843,7 +847,7 @@ void io_live(int dev, int d)
     for (IoBuffers *b : gone) io_delete(b);
 }
 
-// thread t's buffer, allocated by its first use
+// buffer t, allocated by its first use
 hipError_t io_buffer(IoBuffers *b, int t)
 {
     if (!b->buf[t])
@@ -861,7 +865,8 @@ struct IoPlan {
 
 IoPlan io_plan(const s3d_ctx *c, int fields)
 {
-    const long words = (long)(IO_BYTES / sizeof(double)) / fields;
+    const size_t all = sizeof(double) * c->nn * fields;
+    const long words = (long)(std::min(IO_BYTES, std::max(IO_LEAST, all / 8)) / sizeof(double)) / fields;
     IoPlan p;
     if (c->nel * std::min(c->NP, IO_N) <= words) {
         p.ne = c->nel;
@@ -883,10 +888,11 @@ struct IoChunk {
     dim3 grid() const { return dim3((ne + IO_E - 1) / IO_E, (nn + IO_N - 1) / IO_N); }
 };
 
-// Run `one(chunk, buffer, event)` for every chunk on up to IO_THREADS host
-// threads.
-template <typename F>
-int io_chunks(s3d_ctx *c, int fields, F one)
+// For every chunk `start(chunk, buffer, event)`, then `finish` of the same
+// arguments, on up to `most` (at most IO_THREADS) host threads; a thread starts a chunk in its
+// second buffer before it finishes the one in its first.
+template <typename S, typename F>
+int io_chunks(s3d_ctx *c, int fields, int most, S start, F finish)
 {
     const IoPlan p = io_plan(c, fields);
     const long total = p.ce * p.cn;
@@ -895,19 +901,26 @@ int io_chunks(s3d_ctx *c, int fields, F one)
     std::atomic<int> bad(hipSuccess);
     auto work = [&](int t) {
         hipError_t e = hipSetDevice(c->dev);
-        if (e == hipSuccess) e = io_buffer(b, t);
-        for (long q; e == hipSuccess && bad.load() == hipSuccess && (q = next.fetch_add(1)) < total;) {
+        IoChunk k[2];
+        int at = 0, open = 0;   // buffer of the next chunk; chunks started and not finished
+        for (long q; e == hipSuccess && bad.load() == hipSuccess && (q = next.fetch_add(1)) < total; at ^= 1) {
             // consecutive chunks lie side by side in the caller's rows
-            IoChunk k;
-            k.e0 = q % p.ce * p.ne;
-            k.ne = (int)std::min(p.ne, c->nel - k.e0);
-            k.n0 = (int)(q / p.ce) * p.nn;
-            k.nn = std::min(p.nn, c->NP - k.n0);
-            e = one(k, (double *)b->buf[t], b->ev[t]);
+            k[at].e0 = q % p.ce * p.ne;
+            k[at].ne = (int)std::min(p.ne, c->nel - k[at].e0);
+            k[at].n0 = (int)(q / p.ce) * p.nn;
+            k[at].nn = std::min(p.nn, c->NP - k[at].n0);
+            e = io_buffer(b, 2 * t + at);
+            if (e == hipSuccess) e = start(k[at], (double *)b->buf[2 * t + at], b->ev[2 * t + at]);
+            if (e == hipSuccess && ++open == 2) {
+                e = finish(k[at ^ 1], (double *)b->buf[2 * t + (at ^ 1)], b->ev[2 * t + (at ^ 1)]);
+                open = 1;
+            }
         }
+        if (e == hipSuccess && open == 1)
+            e = finish(k[at ^ 1], (double *)b->buf[2 * t + (at ^ 1)], b->ev[2 * t + (at ^ 1)]);
         if (e != hipSuccess) bad.store(e);
     };
-    const int want = (int)std::min<long>({(long)IO_THREADS, total == 1 ? 1 : 1 + total / 2,
+    const int want = (int)std::min<long>({(long)most, 1 + total / IO_PER_THREAD,
                                           std::max(1L, (long)std::thread::hardware_concurrency() / 2)});
     std::vector<std::thread> crew;
     try {
@@ -940,27 +953,38 @@ void io_copy(const s3d_ctx *c, const IoChunk &k, double *field, double *chunk, b
 template <typename Src>
 int io_get(s3d_ctx *c, const Src &src, double *out)
 {
-    return io_chunks(c, 1, [&](const IoChunk &k, double *chunk, hipEvent_t ev) {
-        hipLaunchKernelGGL(export_field<Src>, k.grid(), dim3(256), 0, c->stream, src, k.e0, k.ne, k.n0, k.nn, chunk);
-        hipError_t e = hipGetLastError();
-        if (e == hipSuccess) e = hipEventRecord(ev, c->stream);
-        if (e == hipSuccess) e = hipEventSynchronize(ev);
-        if (e == hipSuccess) io_copy(c, k, out, chunk, true);
-        return e;
-    });
+    return io_chunks(
+        c, 1, IO_THREADS,
+        [&](const IoChunk &k, double *chunk, hipEvent_t ev) {
+            hipLaunchKernelGGL(export_field<Src>, k.grid(), dim3(256), 0, c->stream, src, k.e0, k.ne, k.n0, k.nn, chunk);
+            const hipError_t e = hipGetLastError();
+            return e == hipSuccess ? hipEventRecord(ev, c->stream) : e;
+        },
+        [&](const IoChunk &k, double *chunk, hipEvent_t ev) {
+            const hipError_t e = hipEventSynchronize(ev);
+            if (e == hipSuccess) io_copy(c, k, out, chunk, true);
+            return e;
+        });
 }
+
+// a chunk whose buffer the device reads needs no finish: the buffer's next
+// use waits for it, and io_chunks for the last
+hipError_t io_no_finish(const IoChunk &, double *, hipEvent_t) { return hipSuccess; }
 
 template <typename Dst>
 int io_set(s3d_ctx *c, const Dst &dst, const double *in)
 {
-    return io_chunks(c, 1, [&](const IoChunk &k, double *chunk, hipEvent_t ev) {
-        hipError_t e = hipEventSynchronize(ev);   // the buffer's last chunk
-        if (e != hipSuccess) return e;
-        io_copy(c, k, const_cast<double *>(in), chunk, false);
-        hipLaunchKernelGGL(import_field<Dst>, k.grid(), dim3(256), 0, c->stream, dst, k.e0, k.ne, k.n0, k.nn, chunk);
-        e = hipGetLastError();
-        return e == hipSuccess ? hipEventRecord(ev, c->stream) : e;
-    });
+    return io_chunks(
+        c, 1, 2,
+        [&](const IoChunk &k, double *chunk, hipEvent_t ev) {
+            hipError_t e = hipEventSynchronize(ev);   // the buffer's last chunk
+            if (e != hipSuccess) return e;
+            io_copy(c, k, const_cast<double *>(in), chunk, false);
+            hipLaunchKernelGGL(import_field<Dst>, k.grid(), dim3(256), 0, c->stream, dst, k.e0, k.ne, k.n0, k.nn, chunk);
+            e = hipGetLastError();
+            return e == hipSuccess ? hipEventRecord(ev, c->stream) : e;
+        },
+        io_no_finish);
 }
 
 template <int P, typename R>
@@ -1019,16 +1043,19 @@ struct GradRun {
         for (int q = 0; q < 3; ++q) a.v[q] = unique_src<P, R>(c, c->v[q], c->lo[q]);
         a.inc_dt = inc_dt;
         a.jac = c->jac;
-        return io_chunks(c, 3, [&](const IoChunk &k, double *chunk, hipEvent_t ev) {
-            hipError_t e = hipEventSynchronize(ev);
-            if (e != hipSuccess) return e;
-            for (int q = 0; q < 3; ++q)
-                io_copy(c, k, const_cast<double *>(fw[q]), chunk + (size_t)q * k.ne * k.nn, false);
-            hipLaunchKernelGGL((grad_rho_kernel<P, R>), k.grid(), dim3(256), 0, c->stream, a, k.e0, k.ne, k.n0, k.nn,
-                               chunk);
-            e = hipGetLastError();
-            return e == hipSuccess ? hipEventRecord(ev, c->stream) : e;
-        });
+        return io_chunks(
+            c, 3, 2,
+            [&](const IoChunk &k, double *chunk, hipEvent_t ev) {
+                hipError_t e = hipEventSynchronize(ev);
+                if (e != hipSuccess) return e;
+                for (int q = 0; q < 3; ++q)
+                    io_copy(c, k, const_cast<double *>(fw[q]), chunk + (size_t)q * k.ne * k.nn, false);
+                hipLaunchKernelGGL((grad_rho_kernel<P, R>), k.grid(), dim3(256), 0, c->stream, a, k.e0, k.ne, k.n0,
+                                   k.nn, chunk);
+                e = hipGetLastError();
+                return e == hipSuccess ? hipEventRecord(ev, c->stream) : e;
+            },
+            io_no_finish);
     }
 };
 

@@ -10,8 +10,9 @@ from ses3d_amd import api
 
 pytestmark = pytest.mark.gpu
 
-# order, elements: 4 MB chunks hold 524288 values (174762 of each of three
-# fields): one chunk; rows of 64 nodes; pieces of rows of 27 and of 64 nodes
+# order, elements: chunks of 1 MB to 4 MB hold 131072 to 524288 values (a third
+# of each of three fields): one chunk; rows of 64 nodes; pieces of rows of 27
+# and of 64 nodes
 MESHES = [(7, (3, 2, 2)), (3, (9, 5, 3)), (4, (17, 16, 16)), (2, (33, 32, 20)), (5, (23, 20, 19))]
 
 
