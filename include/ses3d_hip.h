@@ -165,14 +165,12 @@ int s3d_init(s3d_ctx *ctx);
  * src/model_paras.F90:529-561). Requires s3d_init. */
 int s3d_cfl(s3d_ctx *ctx, double *courant);
 
-/* Autotuner: times the element-kernel tile variants (elements per
- * workgroup; FP32 and FP64), the XCD-aware block order, and for FP32 the
- * LDS staging layout and the store order (s3d_set_store_order) on this
- * mesh and keeps the fastest; *tile gets the elements per workgroup chosen
- * and *ms the element kernel time (s3d_get_tuning gives the rest). Needs
- * the state at rest (after s3d_init, before s3d_set_field and s3d_step):
- * the trial launches then leave every field unchanged. No counterpart in
- * the reference. */
+/* Autotuner: times the element kernel's tiles (elements per workgroup) and the
+ * XCD-aware block order on this mesh and keeps the fastest; *tile gets the
+ * elements per workgroup chosen and *ms the element kernel time
+ * (s3d_get_tuning gives the rest). Needs the state at rest (after s3d_init,
+ * before s3d_set_field and s3d_step): the trial launches then leave every
+ * field unchanged. No counterpart in the reference. */
 int s3d_autotune(s3d_ctx *ctx, int *tile, double *ms);
 
 /* Element tile of the step without timing: 0 default, or 1, 2 or 4
@@ -181,25 +179,25 @@ int s3d_autotune(s3d_ctx *ctx, int *tile, double *ms);
  * bit-identical results. No counterpart in the reference. */
 int s3d_set_tile(s3d_ctx *ctx, int tile);
 
-/* LDS layout of the FP32 element kernel without timing: 0 planar (one array
- * per staged component), 1 node-interleaved (the components one contraction
- * term reads in one 16-byte vector). Every layout gives bit-identical
- * results; FP64 and BF16-static simulations use 0. s3d_autotune searches
- * tile x block order x layout. No counterpart in the reference. */
+/* LDS layout of the FP32 element kernel: 0 planar, 1 node-interleaved. The
+ * setting is checked and kept (s3d_get_tuning), and s3d_autotune resets it to
+ * 0, but the kernel has one layout, that of the state block, so it changes
+ * neither results nor speed. FP64 and BF16-static simulations take 0 only. No
+ * counterpart in the reference. */
 int s3d_set_lds_layout(s3d_ctx *ctx, int layout);
 
 /* Where the FP32 element kernel stores the new stress, its compensation and
- * the memory variables: 0 after the weak divergence (default), 1 before it
- * (their registers are then free during the divergence, which raises the
- * occupancy of some GLL orders: order 6 with FP32 compensation of the
- * velocity only runs about 6 % faster). Bit-identical results; planar LDS
- * layout only; FP64 and BF16-static simulations use 0. s3d_autotune
- * searches it with the layout. No counterpart in the reference. */
+ * the memory variables: 0 after the weak divergence (default), 1 before it.
+ * The setting is checked and kept, and s3d_autotune resets it to 0, but the
+ * kernel's order goes by the GLL order and the model, as measured, so it
+ * changes neither results nor speed. Not together with the node-interleaved
+ * layout; FP64 and BF16-static simulations take 0 only. No counterpart in the
+ * reference. */
 int s3d_set_store_order(s3d_ctx *ctx, int early);
 int s3d_get_store_order(s3d_ctx *ctx, int *early);
 
-/* The element tile (elements per workgroup), block order (1: XCD-aware) and
- * LDS layout in use, e.g. as chosen by s3d_autotune. */
+/* The element tile (elements per workgroup) and block order (1: XCD-aware) in
+ * use, e.g. as chosen by s3d_autotune, and the LDS layout setting. */
 int s3d_get_tuning(s3d_ctx *ctx, int *tile, int *xcd_remap, int *lds_layout);
 
 /* GLL points, weights and derivative matrix dl[i + (p+1)*j] = l_i'(xi_j)

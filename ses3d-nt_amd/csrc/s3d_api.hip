@@ -191,7 +191,8 @@ struct s3d_ctx {
          *grad_rho = nullptr,   // FP64 density [nel][NP]
          *dgrad = nullptr,   // FP64 displacement gradient [nel][6][NP], see s3d_enable_displacement_gradient
          *curl_parts = nullptr,   // FP64 [nel][6][NP], see s3d_capture_curl_strain
-         *tr = nullptr, *wdev = nullptr;
+         *tr = nullptr, *wdev = nullptr,
+         *tab = nullptr;   // element-kernel tables, see upload_elem_tables
     double *mm64 = nullptr, *dpx = nullptr, *dpy = nullptr, *dpz = nullptr;
     double bytes = 0;
     // sources
@@ -230,8 +231,8 @@ struct s3d_ctx {
     int nbuf = 2;
     int cur = 0;
     int epb = 0;               // element tile (0 = default), see s3d_autotune
-    int lds_layout = 0;        // LDS staging layout of the FP32 element kernel, see Stage
-    bool early_stores = false; // FP32 element kernel stores the state before the divergence
+    int lds_layout = 0;        // as set by s3d_set_lds_layout
+    bool early_stores = false; // as set by s3d_set_store_order
     int nm = 6;                // memory words per relaxation mechanism (6, or 5: deviatoric)
     int curl_it = -1;          // steps completed at the last s3d_capture_curl_strain
     bool fields_set = false;   // s3d_set_field was called (state not at rest)
@@ -250,9 +251,10 @@ struct s3d_ctx {
 
 namespace {
 
-int dalloc(s3d_ctx *c, void **p, size_t bytes, bool zero = true)
+// pad: bytes past the end that kernels may read (BLOCK_PAD)
+int dalloc(s3d_ctx *c, void **p, size_t bytes, bool zero = true, size_t pad = 0)
 {
-    hipError_t e = hipMalloc(p, bytes ? bytes : 16);
+    hipError_t e = hipMalloc(p, (bytes ? bytes : 16) + pad);
     if (e != hipSuccess) {
         *p = nullptr;
         return fail("hipMalloc(" + std::to_string(bytes) + " B): " + hipGetErrorString(e));
@@ -315,7 +317,7 @@ int alloc_state(s3d_ctx *c)
     // components and are not separate allocations
     c->ns = state_components(c->o.kahan_sigma, c->visco ? c->nm : 0);
     for (int k = 0; k < c->nbuf; ++k)
-        if (dalloc(c, &c->blk[k], rs * c->ns * c->nn)) return 1;
+        if (dalloc(c, &c->blk[k], rs * c->ns * c->nn, true, BLOCK_PAD)) return 1;
     set_state_block(c, 0);
     if (dalloc(c, &c->force, rs * 3 * c->nn, false)) return 1;
     if (dalloc(c, (void **)&c->d_it, sizeof(int))) return 1;
@@ -347,16 +349,45 @@ int upload_tables(s3d_ctx *c, const std::vector<double> &sin1)
     return 0;
 }
 
+// The element kernel's tables (ElemArgs::coef, gx, gz), FP64.
+int upload_elem_tables(s3d_ctx *c, const std::vector<double> &sin1)
+{
+    const int P1 = c->P1;
+    std::vector<double> t;
+    t.reserve(coef_words(P1) + 4 * P1 * (c->g.nx + c->g.nz));
+    // dl(q,i) = l_q'(xi_i) is stored at c->dl[q + P1*i]
+    for (double d : {c->dx, c->dy, c->dz})
+        for (int i = 0; i < P1; ++i)
+            for (int q = 0; q < P1; ++q) t.push_back(2.0 * c->dl[q + P1 * i] / d);
+    for (int i = 0; i < P1; ++i)
+        for (int q = 0; q < P1; ++q) t.push_back(c->dl[i + P1 * q] * c->weights[q]);
+    t.insert(t.end(), c->weights, c->weights + P1);
+    for (int e = 0; e < c->g.nx; ++e) {
+        const double *s = &sin1[(size_t)e * P1], *x = &c->x1[(size_t)e * P1], *p = &c->px1[(size_t)e * P1];
+        t.insert(t.end(), s, s + P1);
+        for (int q = 0; q < P1; ++q) t.push_back(1.0 / s[q]);
+        for (int q = 0; q < P1; ++q) t.push_back(std::cos(x[q]) / s[q]);
+        t.insert(t.end(), p, p + P1);
+    }
+    for (int e = 0; e < c->g.nz; ++e) {
+        const double *r = &c->z1[(size_t)e * P1], *p = &c->pz1[(size_t)e * P1];
+        t.insert(t.end(), r, r + P1);
+        for (int q = 0; q < P1; ++q) t.push_back(1.0 / r[q]);
+        for (int q = 0; q < P1; ++q) t.push_back(r[q] * r[q]);
+        t.insert(t.end(), p, p + P1);
+    }
+    if (dalloc(c, &c->tab, sizeof(double) * t.size(), false)) return 1;
+    HIPCHK(hipMemcpy(c->tab, t.data(), sizeof(double) * t.size(), hipMemcpyHostToDevice));
+    return 0;
+}
+
 size_t rsize(const s3d_ctx *c) { return c->fp32 ? sizeof(float) : sizeof(double); }
 
-// the element kernel's variant (elem_body's LL) for the layout and store order
 // the velocity compensation arrays as FP32 or BF16 words (null when the
 // simulation keeps the other kind or none)
 template <typename R>
 R *lo32(const s3d_ctx *c, int q) { return c->kv == 1 ? (R *)c->lo[q] : nullptr; }
 bf16 *lo16(const s3d_ctx *c, int q) { return c->kv == 2 ? (bf16 *)c->lo[q] : nullptr; }
-
-int kernel_variant(const s3d_ctx *c) { return c->early_stores ? 2 : c->lds_layout; }
 
 inline unsigned nblocks(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
@@ -400,9 +431,11 @@ ElemArgs<R> elem_args(s3d_ctx *c, int rd = -1, int wr = -1)
     a.dgrad = (decltype(a.dgrad))(c->dgrad);
     a.dt = c->g.dt;
     using C = coef_t<R>;
-    a.tth = (decltype(a.tth))((const ThTab<C> *)c->tth);
-    a.tr = (decltype(a.tr))((const RTab<C> *)c->tr);
-    a.px = (decltype(a.px))(c->dpx); a.py = (decltype(a.py))(c->dpy); a.pz = (decltype(a.pz))(c->dpz);
+    const double *tab = (const double *)c->tab;
+    a.coef = (decltype(a.coef))(tab);
+    a.gx = (decltype(a.gx))(tab + coef_words(P1));
+    a.gz = (decltype(a.gz))(tab + coef_words(P1) + 4 * P1 * c->g.nx);
+    a.py = (decltype(a.py))(c->dpy);
     a.alpha = c->g.taper_slope;
     a.taper_on = c->g.taper_width > 0;
     a.src_slot = (decltype(a.src_slot))(c->d_slot);
@@ -413,15 +446,6 @@ ElemArgs<R> elem_args(s3d_ctx *c, int rd = -1, int wr = -1)
     a.d2 = (C)((2.0 / c->dy) * c->jac);
     a.d3 = (C)(-((2.0 / c->dz) * c->jac));
     for (int m = 0; m < NRDISS; ++m) a.rate[m] = (R)(c->g.dt / TAU_P[m]);
-    for (int q = 0; q < P1; ++q) a.w[q] = (C)c->weights[q];
-    for (int i = 0; i < P1; ++i)
-        for (int q = 0; q < P1; ++q) {
-            // dl(q,i) = l_q'(xi_i) is stored at c->dl[q + P1*i]
-            a.Dx[i * P1 + q] = (C)(2.0 * c->dl[q + P1 * i] / c->dx);
-            a.Dy[i * P1 + q] = (C)(2.0 * c->dl[q + P1 * i] / c->dy);
-            a.Dz[i * P1 + q] = (C)(2.0 * c->dl[q + P1 * i] / c->dz);
-            a.dlw[i * P1 + q] = (C)(c->dl[i + P1 * q] * c->weights[q]);
-        }
     return a;
 }
 
@@ -493,7 +517,6 @@ int launch_elem(s3d_ctx *c, const ElemArgs<R> &ea, const RecArgs<R> &ra, hipStre
     l.nel = c->nel;
     l.vm = c->visco ? c->nm : 0;
     l.ks = c->o.kahan_sigma;
-    l.ll = kernel_variant(c);
     l.bf16_static = c->o.bf16_static;
     l.epb = epb;
     const hipError_t e = launch_elem_kernel<P, R>(l, ea, ra, st);
@@ -516,7 +539,7 @@ std::vector<int> tile_candidates(bool bf16_static)
 
 void drop_graph(s3d_ctx *c);
 
-// Time every tile variant x block order on this mesh (state at rest, so
+// Time every tile x block order on this mesh (state at rest, so
 // the trial launches write zeros over zeros) and keep the fastest.
 template <int P, typename R>
 int autotune_p(s3d_ctx *c, int *tile_out, double *ms_out)
@@ -525,38 +548,33 @@ int autotune_p(s3d_ctx *c, int *tile_out, double *ms_out)
     HIPCHK(hipEventCreate(&e0));
     HIPCHK(hipEventCreate(&e1));
     double best = 1e300;
-    int best_tile = c->epb, best_remap = c->o.xcd_remap, best_ll = kernel_variant(c);
-    const int nll = (c->fp32 && !c->o.bf16_static) ? 3 : 1;
+    int best_tile = c->epb, best_remap = c->o.xcd_remap;
     for (int tile : tile_candidates<P>(c->o.bf16_static))
-        for (int ll = 0; ll < nll; ++ll)
-            for (int remap = 0; remap < 2; ++remap) {
-                c->o.xcd_remap = remap;
-                c->lds_layout = ll == 1 ? 1 : 0;
-                c->early_stores = ll == 2;
-                ElemArgs<R> ea = elem_args<P, R>(c);
-                RecArgs<R> none = rec_args<R>(c);
-                none.n = 0;
-                if (int rc = launch_elem<P, R>(c, ea, none, c->stream, tile)) return rc;   // warm-up
-                HIPCHK(hipEventRecord(e0, c->stream));
-                for (int r = 0; r < 3; ++r)
-                    if (int rc = launch_elem<P, R>(c, ea, none, c->stream, tile)) return rc;
-                HIPCHK(hipEventRecord(e1, c->stream));
-                HIPCHK(hipEventSynchronize(e1));
-                float ms = 0.f;
-                HIPCHK(hipEventElapsedTime(&ms, e0, e1));
-                if (ms / 3.0 < best) {
-                    best = ms / 3.0;
-                    best_tile = tile;
-                    best_remap = remap;
-                    best_ll = ll;
-                }
+        for (int remap = 0; remap < 2; ++remap) {
+            c->o.xcd_remap = remap;
+            ElemArgs<R> ea = elem_args<P, R>(c);
+            RecArgs<R> none = rec_args<R>(c);
+            none.n = 0;
+            if (int rc = launch_elem<P, R>(c, ea, none, c->stream, tile)) return rc;   // warm-up
+            HIPCHK(hipEventRecord(e0, c->stream));
+            for (int r = 0; r < 3; ++r)
+                if (int rc = launch_elem<P, R>(c, ea, none, c->stream, tile)) return rc;
+            HIPCHK(hipEventRecord(e1, c->stream));
+            HIPCHK(hipEventSynchronize(e1));
+            float ms = 0.f;
+            HIPCHK(hipEventElapsedTime(&ms, e0, e1));
+            if (ms / 3.0 < best) {
+                best = ms / 3.0;
+                best_tile = tile;
+                best_remap = remap;
             }
+        }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     c->epb = best_tile;
     c->o.xcd_remap = best_remap;
-    c->lds_layout = best_ll == 1 ? 1 : 0;
-    c->early_stores = best_ll == 2;
+    c->lds_layout = 0;
+    c->early_stores = false;
     drop_graph(c);
     if (tile_out) *tile_out = best_tile == 0 ? default_epb<P>() : best_tile;
     if (ms_out) *ms_out = best;
@@ -1244,7 +1262,6 @@ int upload_receivers(s3d_ctx *c)
 struct BatchGroup {
     int p = 0;
     int epb = 0;
-    int ll = 0;                 // element kernel variant (elem_body's LL)
     int ks = 0;                 // stress compensation mode
     int vm = 0;                 // memory words per mechanism (0 elastic, 6, 5)
     int kv = 0;                 // velocity compensation words (0, 1 FP32, 2 BF16)
@@ -1362,7 +1379,6 @@ int batch_launch_group(const BatchGroup &G, bool first, hipStream_t st)
     l.rown = G.d_rown;
     l.vm = G.vm;
     l.ks = G.ks;
-    l.ll = G.ll;
     l.epb = G.epb;
     l.nwg = (unsigned)G.ewg;
     l.args = (const ElemArgs<R> *)G.d_eargs + (size_t)G.phase * n;
@@ -1497,7 +1513,6 @@ int batch_build(s3d_batch *b)
         for (const s3d_ctx *c : G.sims)
             if (c->nel > big->nel) big = c;
         G.epb = big->epb;
-        G.ll = big->fp32 ? kernel_variant(big) : 0;
         G.ride = true;
         for (const s3d_ctx *c : G.sims) G.ride = G.ride && (c->nrec_dev == 0 || receivers_ride(c));
     }
@@ -1646,7 +1661,7 @@ int s3d_destroy(s3d_ctx *c)
     if (c->model) {
         // the static fields belong to the model's simulation
         void **shared[] = {&c->dt_inv_mm, (void **)&c->mm64, &c->lam, &c->mu, &c->tau, &c->rho, &c->ca,
-                           &c->cb, &c->cc, &c->tth, &c->tr, &c->wdev, (void **)&c->dpx,
+                           &c->cb, &c->cc, &c->tth, &c->tr, &c->wdev, &c->tab, (void **)&c->dpx,
                            (void **)&c->dpy, (void **)&c->dpz};
         for (void **q : shared) *q = nullptr;
         c->model->sharers--;
@@ -1656,7 +1671,7 @@ int s3d_destroy(s3d_ctx *c)
     c->sig = c->sig_lo = c->mem = nullptr;   // views of the state blocks
     void *bufs[] = {c->v[0], c->v[1], c->v[2], c->lo[0], c->lo[1], c->lo[2], c->dt_inv_mm, c->blk[0], c->blk[1],
                     c->mat, c->rho, c->ca, c->cb, c->cc, c->grad_rho, c->dgrad, c->curl_parts,
-                    c->force, c->tth, c->tr, c->wdev, c->mm64, c->dpx, c->dpy, c->dpz,
+                    c->force, c->tth, c->tr, c->wdev, c->tab, c->mm64, c->dpx, c->dpy, c->dpz,
                     c->d_slot, c->d_chan, c->d_coef, c->d_stf, c->d_rec_e, c->d_rec_nch,
                     c->d_rec_off, c->d_rec_ch, c->d_rec_vm, c->d_traces, c->d_rec_rot, c->d_rot_e, c->d_rot_buf};
     for (void *b : bufs) dfree(b);
@@ -1706,7 +1721,7 @@ int s3d_create_shared(s3d_ctx *base, s3d_ctx **out)
     // static fields: the model's, not copied
     c->dt_inv_mm = m->dt_inv_mm; c->mm64 = m->mm64; c->lam = m->lam; c->mu = m->mu; c->tau = m->tau;
     c->rho = m->rho; c->ca = m->ca; c->cb = m->cb; c->cc = m->cc; c->tth = m->tth; c->tr = m->tr;
-    c->wdev = m->wdev; c->dpx = m->dpx; c->dpy = m->dpy; c->dpz = m->dpz;
+    c->wdev = m->wdev; c->tab = m->tab; c->dpx = m->dpx; c->dpy = m->dpy; c->dpz = m->dpz;
     c->model = m;
     m->sharers++;
     io_live(c->dev, 1);
@@ -1843,6 +1858,7 @@ int s3d_init(s3d_ctx *c)
     std::vector<double> sin1(g.nx * P1), th1 = c->x1, ph1 = c->y1, r1 = c->z1;
     for (size_t q = 0; q < sin1.size(); ++q) sin1[q] = std::sin(c->x1[q]);
     if (c->fp32 ? upload_tables<coef_t<float>>(c, sin1) : upload_tables<double>(c, sin1)) return 1;
+    if (upload_elem_tables(c, sin1)) return 1;
     {
         if (dalloc(c, &c->wdev, sizeof(double) * P1)) return 1;
         HIPCHK(hipMemcpy(c->wdev, c->weights, sizeof(double) * P1, hipMemcpyHostToDevice));
@@ -1875,7 +1891,7 @@ int s3d_init(s3d_ctx *c)
     // lam, mu (and tau) as one element-major block; lam/mu/tau point at the
     // components' first entries
     const int ncm = c->visco ? 3 : 2;
-    if (dalloc(c, &c->mat, ss * ncm * c->nn, false)) return 1;
+    if (dalloc(c, &c->mat, ss * ncm * c->nn, false, BLOCK_PAD)) return 1;
     c->lam = c->mat;
     c->mu = (char *)c->mat + ss * c->NP;
     c->tau = c->visco ? (char *)c->mat + 2 * ss * c->NP : nullptr;

@@ -76,110 +76,6 @@ __device__ inline void kahan_add(R &s, R &c, R inc)
 // ---------------------------------------------------------------------------
 // element kernel
 // ---------------------------------------------------------------------------
-// Direct HBM -> LDS load of one dword per lane (global_load_lds_dword):
-// lane l writes LDS byte address lds + 4 l. Written as inline assembly so the
-// compiler's wait accounting never sees it: callers issue these loads before
-// any compiler-issued load (vector memory operations complete in issue
-// order, so the compiler's own waits stay exact) and read the LDS words
-// only after wait_vmem_zero. The statement writes M0, so M0 is in its clobber
-// list: the compiler keeps nothing there across it. LLVM reserves M0 and warns
-// about the clobber; in the gfx950 code of this library the only
-// instructions that touch M0 are these statements' own.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void lds_dma_dword(const void *g, unsigned lds)
-{
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
-                 :: "v"(g), "s"(__builtin_amdgcn_readfirstlane(lds)) : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
-// s_waitcnt vmcnt(0), returning a zero that the reads of LDS words written by
-// lds_dma_dword must add to their index: the data dependency orders those
-// reads after the wait without a memory clobber (which would make the
-// compiler reload every argument read through a pointer).
-__device__ __forceinline__ int wait_vmem_zero()
-{
-    int z;
-    asm volatile("s_waitcnt vmcnt(0)\n\tv_mov_b32 %0, 0" : "=v"(z));
-    return z;
-}
-
-typedef float lds4 __attribute__((ext_vector_type(4)));
-
-// LDS layout of the tile's staged velocity and effective stress (the
-// autotuner's choice; every layout gives the same arithmetic):
-//   LL = 0  planar: lds[c][node], one 4-byte read per component;
-//   LL = 1  node-interleaved (FP32 only): 48 bytes per node, the velocity in
-//           the first 16-byte vector and the stress as the three triples the
-//           divergence contracts, (xx xy xz | xy yy yz | xz yz zz), one
-//           16-byte read per contraction term instead of three 4-byte reads.
-template <typename R, int LL, int N>
-struct Stage {
-    static constexpr bool INTERLEAVED = LL == 1 && sizeof(R) == 4;
-    R planar[INTERLEAVED ? 1 : 6][INTERLEAVED ? 1 : N];
-    lds4 inter[INTERLEAVED ? N : 1][INTERLEAVED ? 3 : 1];
-
-    __device__ void put_v(int n, R v0, R v1, R v2)
-    {
-        if constexpr (INTERLEAVED) {
-            inter[n][0] = (lds4){v0, v1, v2, 0.f};
-        } else {
-            planar[0][n] = v0;
-            planar[1][n] = v1;
-            planar[2][n] = v2;
-        }
-    }
-    // velocity components at node n
-    __device__ void get_v(int n, R *v) const
-    {
-        if constexpr (INTERLEAVED) {
-            const lds4 w = inter[n][0];
-            v[0] = w.x; v[1] = w.y; v[2] = w.z;
-        } else {
-            v[0] = planar[0][n]; v[1] = planar[1][n]; v[2] = planar[2][n];
-        }
-    }
-    // effective stress s[xx xy xz yy yz zz]
-    __device__ void put_s(int n, const R *sv)
-    {
-        if constexpr (INTERLEAVED) {
-            inter[n][0] = (lds4){sv[XX], sv[XY], sv[XZ], 0.f};
-            inter[n][1] = (lds4){sv[XY], sv[YY], sv[YZ], 0.f};
-            inter[n][2] = (lds4){sv[XZ], sv[YZ], sv[ZZ], 0.f};
-        } else {
-#pragma unroll
-            for (int c = 0; c < 6; ++c) planar[c][n] = sv[c];
-        }
-    }
-    // the stress components that contraction d (0 theta, 1 phi, 2 r) reads at
-    // node n: (xx xy xz), (xy yy yz), (xz yz zz)
-    __device__ void get_s(int d, int n, R *w3) const
-    {
-        if constexpr (INTERLEAVED) {
-            const lds4 w = inter[n][d];
-            w3[0] = w.x; w3[1] = w.y; w3[2] = w.z;
-        } else {
-            constexpr int comp[3][3] = {{XX, XY, XZ}, {XY, YY, YZ}, {XZ, YZ, ZZ}};
-            w3[0] = planar[comp[d][0]][n];
-            w3[1] = planar[comp[d][1]][n];
-            w3[2] = planar[comp[d][2]][n];
-        }
-    }
-};
-
-// Per-lane state of one element tile (EPB elements, one lane per
-// element-local node). VM: memory words per mechanism (state_components).
-template <typename R, int VM>
-struct TileState {
-    R v[3];             // velocity gathered from the unique nodes
-    R sg[6];            // stress
-    R lam, mu, tau;     // dt-scaled moduli, tau
-    R M[VM ? NRDISS * VM : 1];
-    R lo[6];            // stress compensation, kahan_sigma 1
-    unsigned lo2[3];    // stress compensation, kahan_sigma 2 (packed BF16 pairs)
-};
-
 // Element-major block fields (the state block, lam/mu/tau, the displacement
 // gradient; the element force has its own two-part layout, force_index):
 // component c of element e occupies the NP entries at (e * nc + c) * NP.
@@ -203,461 +99,539 @@ __device__ __forceinline__ long force_index(long e, int c, int node, long nel)
     return node < NM ? (e * 3 + c) * NM + node : nel * 3 * NM + (e * 3 + c) * NL + (node - NM);
 }
 
-// Issue the loads of tile `tile` into `s` (no waits). Lanes without an
-// element (the tail of the last tile) read element 0's addresses, so every
-// load is unconditional and in bounds; such lanes store nothing. KS: stress
-// compensation 0 off, 1 FP32 words, 2 BF16 words in pairs (a template
-// parameter: a run-time choice leaves register joins that wait for every
-// load in flight).
-template <int P, int E, typename R, int VM, bool S16, bool LOADM, int KS>
-__device__ __forceinline__ void load_tile(const ElemArgs<R> &a, int tile, TileState<R, VM> &s)
+// Direct HBM -> LDS loads (global_load_lds): the lanes of a wave write
+// consecutive LDS words or 16-byte vectors from byte address `lds` (the same in
+// the wave) on. Written as inline assembly so the compiler's wait accounting
+// never sees them: it would wait for all of them before any read of LDS.
+// Vector memory operations complete in issue order, and wait_loads<N> waits
+// until at most the N newest are outstanding. The statements write M0, so it
+// is in their clobber list; LLVM reserves M0 and warns about the clobber.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void lds_load_dword(const void *g, unsigned lds)
 {
-    using S = Shape<P, E>;
-    constexpr int P1 = S::P1, NP = S::NP, EPB = S::EPB;
-    constexpr int NS = state_components(KS, VM);
-    constexpr bool VISCO = VM != 0;
-    const int t = threadIdx.x;
-    const int slot = t / NP;
-    const int node = t - slot * NP;
-    const int e = tile * EPB + slot;
-    const bool valid = slot < EPB && e < a.nel;
-    const int ee = valid ? e : 0;
-    const int ex = ee % a.nx, ey = (ee / a.nx) % a.ny, ez = ee / (a.nx * a.ny);
-    const int i = node % P1, j = (node / P1) % P1, k = node / (P1 * P1);
-    const long u = unique_index<P>(ex, ey, ez, i, j, k, a.nx, a.ny);
-    s.v[0] = a.vx[u];
-    s.v[1] = a.vy[u];
-    s.v[2] = a.vz[u];
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
+                 :: "v"(g), "s"(__builtin_amdgcn_readfirstlane(lds)) : "m0");
+}
+
+__device__ __forceinline__ void lds_load_x4(const void *g, unsigned lds)
+{
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+                 :: "v"(g), "s"(__builtin_amdgcn_readfirstlane(lds)) : "m0");
+}
+#pragma clang diagnostic pop
+
+template <int N>
+__device__ __forceinline__ void wait_loads()
+{
+    static_assert(N < 64, "vmcnt has 6 bits");
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
+}
+
+__device__ __forceinline__ unsigned lds_address(const void *p) { return (unsigned)(size_t)p; }
+
+// The words [w0, w0 + n) of an element-major block into LDS, in 16-byte
+// vectors by the workgroup's NT lanes, n at most W. The block starts on a
+// 16-byte boundary and the vectors do too: word w0 arrives at lds[w0 & 3], and
+// up to 3 words before and after the range come along (the blocks are
+// allocated BLOCK_PAD bytes longer). lds holds lds_words(W).
+constexpr int lds_words(int W) { return (W + 3 + 3) / 4 * 4; }
+
+// loads that every wave issues for a whole run of W words (some issue more)
+constexpr int run_loads(int W, int NT) { return W > 4 * NT - 256 ? (W - 4 * NT + 256 + 4 * NT - 1) / (4 * NT) : 0; }
+
+template <int W, int NT>
+__device__ __forceinline__ int lds_load_run(const float *block, long w0, int n, const float *lds)
+{
+    const int off = (int)(w0 & 3), end = n > 0 ? n + off : 0;
+    const int lane = threadIdx.x & 63, first = (threadIdx.x >> 6) * 256;
+    const float *src = block + (w0 - off);
 #pragma unroll
-    for (int c = 0; c < 6; ++c) s.sg[c] = a.sig[em_index(ee, NS, c, NP, node)];
-    s.tau = R(0);
-    // lam, mu (, tau): one element-major block, the pointers at its components
-    const long mb = em_index(ee, VISCO ? 3 : 2, 0, NP, node);
-    if constexpr (S16) {
-        s.lam = (R)(float)a.s16.lam[mb];
-        s.mu = (R)(float)a.s16.mu[mb];
-        if constexpr (VISCO) s.tau = (R)(float)a.s16.tau[mb];
-    } else {
-        s.lam = a.lam[mb];
-        s.mu = a.mu[mb];
-        if constexpr (VISCO) s.tau = a.tau[mb];
+    for (int q = 0; q < (W + 3 + 4 * NT - 1) / (4 * NT); ++q) {
+        const int at = first + q * 4 * NT;
+        if (at + 4 * lane < end) lds_load_x4(src + at + 4 * lane, lds_address(lds + at));
     }
-    if constexpr (VISCO && LOADM) {
+    return off;
+}
+
+// Geometry rows per element (FP64): sin, 1/sin, cot of theta_q and the theta
+// taper profile (ElemArgs::gx), the phi profile (py), r, 1/r, r^2 of r_q and the
+// r profile (gz).
+enum { G_SIN = 0, G_ISIN, G_COT, G_PX, G_PY, G_R, G_IR, G_R2, G_PZ, G_N };
+
+// The tables of a tile into LDS, word by word: the coefficients (CoefTable
+// order) and the geometry rows of its elements, [EPB][G_N][P1] doubles.
+template <int P, int EPB, int NT, typename R>
+__device__ __forceinline__ void load_tables(const ElemArgs<R> &a, int tile, const double *cf, const double *gtab)
+{
+    constexpr int P1 = P + 1, CW = 2 * coef_words(P1), GW = 2 * G_N * P1;
+    const int t = threadIdx.x, w = t & ~63;
+    const unsigned *coef = (const unsigned *)(const double *)a.coef;
 #pragma unroll
-        for (int c = 0; c < NRDISS * VM; ++c) s.M[c] = a.mem[em_index(ee, NS, c, NP, node)];
-    }
+    for (int q = 0; q < (CW + NT - 1) / NT; ++q)
+        if (q * NT + t < CW) lds_load_dword(coef + q * NT + t, lds_address((const unsigned *)cf + q * NT + w));
 #pragma unroll
-    for (int c = 0; c < 6; ++c) s.lo[c] = R(0);
-#pragma unroll
-    for (int q = 0; q < 3; ++q) s.lo2[q] = 0u;
-    if constexpr (KS == 2) {
-#pragma unroll
-        for (int q = 0; q < 3; ++q) s.lo2[q] = a.sig_lo2[em_index(ee, NS, q, NP, node)];
-    } else if constexpr (KS == 1) {
-#pragma unroll
-        for (int c = 0; c < 6; ++c) s.lo[c] = a.sig_lo[em_index(ee, NS, c, NP, node)];
+    for (int q = 0; q < (EPB * GW + NT - 1) / NT; ++q) {
+        const int at = q * NT + t;
+        if (at < EPB * GW) {
+            const int es = at / GW, m = at - es * GW, row = m / (2 * P1), m2 = m - row * 2 * P1;
+            int e = tile * EPB + es;
+            e = e < a.nel ? e : a.nel - 1;
+            const int ex = e % a.nx, ey = (e / a.nx) % a.ny, ez = e / (a.nx * a.ny);
+            const double *x = row < G_PY ? (const double *)a.gx + (ex * 4 + row) * P1
+                              : row == G_PY ? (const double *)a.py + ey * P1
+                                            : (const double *)a.gz + (ez * 4 + row - G_R) * P1;
+            lds_load_dword((const unsigned *)x + m2, lds_address((const unsigned *)gtab + q * NT + w));
+        }
     }
 }
 
-// Geometry rows per element (FP64): sin, 1/sin, cot of theta_q; r, 1/r, r^2
-// of r_q; the three taper profiles.
-enum { G_SIN = 0, G_ISIN, G_COT, G_R, G_IR, G_R2, G_PX, G_PY, G_PZ, G_N };
+// Data of one tile. FP32 kernels keep it in LDS: the state [EPB][NS][NP], the
+// moduli [EPB][NC][NP] (not BF16 ones), the velocity [3][NT]; FP64 kernels in
+// registers, with LDS for the staged velocity, then effective stress.
+template <int P, int E, typename R, int VM, bool S16, int KS>
+struct Tile {
+    using S = Shape<P, E>;
+    static constexpr bool DMA = sizeof(R) == 4, MAT = DMA && !S16;
+    static constexpr int NS = state_components(KS, VM), NC = VM ? 3 : 2;
+    static constexpr int TW = S::EPB * NS * S::NP, MW = S::EPB * NC * S::NP;   // words
+    static constexpr int SBUF = DMA ? lds_words(TW) : 6 * S::EPB * S::NP, MBUF = MAT ? lds_words(MW) : 1,
+                         VBUF = DMA ? 3 * S::NT : 1;
+    static constexpr int LDS = (int)sizeof(R) * (SBUF + MBUF + VBUF) +
+                               8 * (coef_words(S::P1) + S::EPB * G_N * S::P1) + 4 * S::EPB;
+};
 
-// Element kernel body: the workgroup advances tile `blk` (EPB elements, one
+// Where the kernel stores the new stress, compensation and memory variables:
+// before the weak divergence, while other waves still compute, or after it.
+// Early costs registers nothing (the values leave before the divergence needs
+// its own) and starts the stores sooner, at orders up to 5 and for elastic
+// order 6: order 5 383 us against 393 at 48x40x24 with five memory words,
+// 260 against 295 elastic with FP32 compensation; order 3 elastic 108 against
+// 117 at 61x53x31; order 2 698 against 725 at 100x100x64. The wide
+// workgroups of orders 6 and 7 are few on a CU and wait for their own stores
+// at the divergence's barrier: order 6 440 us late, 490 early at 40x36x20,
+// order 7 397 and 421 at 36x30x18 (elastic 277 and 287).
+template <int P, typename R, int VM>
+constexpr bool stores_early() { return sizeof(R) == 4 && (P <= 5 || (P == 6 && VM == 0)); }
+
+// Dynamic LDS of a launch, which the kernel does not use: it keeps the
+// workgroups of a CU to about 130 KB of tiles in flight. More of them only
+// widen the window of memory that is open at a time: order 4, 32 KB a tile, 5
+// and 4 workgroups per CU: 2.25 and 2.16 ms at 96x96x48 with five memory
+// words and BF16 compensation, 1.50 and 1.43 ms at 96x96x32 with six and none;
+// 3 workgroups 2.22 ms.
+template <int P, int E, typename R, int VM, bool S16, int KS>
+constexpr unsigned spare_lds()
+{
+    constexpr int cu = 160 * 1024, lds = Tile<P, E, R, VM, S16, KS>::LDS;
+    constexpr int fit = cu / lds, want = 130 * 1024 / lds > 2 ? 130 * 1024 / lds : 2;
+    return Tile<P, E, R, VM, S16, KS>::DMA && fit > want ? cu / (want + 1) + 1 - lds : 0;
+}
+
+// Element kernel body: the workgroup advances tile `tile` (EPB elements, one
 // lane per element-local node). S16: the static per-node fields are stored
-// in BF16 (ElemArgs::s16). KS: stress compensation (see load_tile). LL: the
-// kernel variant, 0 planar LDS staging, 1 node-interleaved staging (see
-// Stage), 2 planar staging with the new stress, compensation and memory
-// variables stored before the weak divergence instead of after it (their
-// registers are then free during the divergence, which raises the occupancy
-// of some orders and compensation modes); the arithmetic is the same. VM:
-// memory words per mechanism, 0 elastic, 6 the six components, 5 their
-// deviatoric part (see the stress rate below).
-template <int P, int E, typename R, int VM, bool S16, int KS, int LL>
-__device__ __forceinline__ void elem_body(const ElemArgs<R> &a, int blk)
+// in BF16 (ElemArgs::s16). KS: stress compensation, 0 off, 1 FP32 words, 2
+// BF16 words in pairs (a template parameter: a run-time choice leaves register
+// joins that wait for every load in flight). VM: memory words per mechanism, 0
+// elastic, 6 the six components, 5 their deviatoric part (see the stress rate
+// below).
+//
+// FP32 kernels load everything straight into LDS: the tables and the velocity
+// first, for the strain rate, behind them the tile's part of the state block
+// and of the moduli, which are contiguous, in 16-byte vectors. They hold no
+// state in registers until they use it, and the effective stress takes the
+// place of the stress in LDS. HBM bounds them (the contractions only at order
+// 6): one dword load per lane and component into registers, waiting for the
+// lot, ran 2.46 ms at order 4, 96x96x48 with five memory words and BF16
+// compensation (5.0 TB/s with the force), this 2.07 ms (5.9 TB/s; a copy
+// reaches 6.2); order 2, 100x100x64 0.86 and 0.68 ms; order 3, 100x100x50 1.28
+// and 1.15; order 5, 48x40x24 0.46 and 0.39; order 6, 40x36x20 0.55 and 0.48;
+// order 7, 36x30x18 0.44 and 0.40. (The part of these gains that is the
+// workgroup order's is at chunk_block.) FP64 kernels keep the tile in
+// registers, since in LDS it would leave one workgroup per CU: 0.53 ms at
+// order 4, 48x48x24, 5.8 TB/s.
+template <int P, int E, typename R, int VM, bool S16, int KS>
+__device__ __forceinline__ void elem_body(const ElemArgs<R> &a, int tile)
 {
     using S = Shape<P, E>;
     using C = coef_t<R>;
-    constexpr int P1 = S::P1, NP = S::NP, EPB = S::EPB, NE = EPB;
-    constexpr int NS = state_components(KS, VM);
+    constexpr int P1 = S::P1, NP = S::NP, EPB = S::EPB, NT = S::NT;
+    using T = Tile<P, E, R, VM, S16, KS>;
+    constexpr int NS = T::NS;         // words per node of the state block
     constexpr bool VISCO = VM != 0;
     constexpr int NM = NRDISS * VM;   // memory words per node
-    constexpr bool EARLY = LL == 2;
-    __shared__ Stage<R, LL == 1 ? 1 : 0, EPB * NP> lds;
-    __shared__ C cf[4][P1 * P1];     // Dx, Dy, Dz, dl*w
-    __shared__ C cw[P1];             // GLL weights
-    __shared__ C gtab[NE][G_N * P1]; // geometry rows of the tile's elements
-    __shared__ int sst[NE];          // moment-tensor source slot per element
+    constexpr int NC = T::NC;         // lam, mu (, tau)
+    constexpr bool DMA = T::DMA, MAT = T::MAT;
+    constexpr int TW = T::TW, MW = T::MW;
+    constexpr bool EARLY = stores_early<P, R, VM>();
+    __shared__ __align__(16) R sbuf[T::SBUF];
+    __shared__ __align__(16) R mbuf[T::MBUF];
+    __shared__ R vbuf[T::VBUF];
+    static_assert(sizeof(C) == 8, "tables are FP64");
+    __shared__ __align__(16) C cf[coef_words(P1)];    // Dx, Dy, Dz, dl*w, weights
+    __shared__ __align__(16) C gtab[EPB][G_N * P1];   // geometry rows of the tile's elements
+    __shared__ int sst[EPB];                          // moment-tensor source slot per element
 
     const int t = threadIdx.x;
     const int slot = t / NP;
     const int node = t - slot * NP;
     const bool inside = slot < EPB;
+    const int es = inside ? slot : 0;
     const int i = node % P1, j = (node / P1) % P1, k = node / (P1 * P1);
-    const int L = (inside ? slot : 0) * NP;
-    const int tile0 = blk;
+    // element of this lane; lanes without one (the tail of the last tile, or
+    // past the tile's nodes) read element 0's addresses and store nothing
+    const int e = tile * EPB + slot;
+    const bool valid = inside && e < a.nel;
+    const long ev = valid ? e : 0;
+    const long eb = ev * NP + node;   // element-local address
 
-    // ---- memory variables of the FP32 kernels: streamed straight into LDS
-    // (lane t's words at mbuf[c][t]), so they hold no registers until the
-    // stress rate; issued before every other load ----
-    constexpr bool MDMA = VISCO && sizeof(R) == 4;
-    __shared__ R mbuf[MDMA ? NM : 1][MDMA ? S::NT : 1];
-    if constexpr (MDMA) {
-        // operands in registers first: each asm statement clobbers memory,
-        // and argument blocks read through a pointer would be reloaded
-        const int e = tile0 * EPB + slot;
-        const R *mem = a.mem + em_index((inside && e < a.nel) ? e : 0, NS, 0, NP, node);
-        const unsigned base = (unsigned)(size_t)&mbuf[0][(t >> 6) << 6];
+    // ---- loads: what the strain rate needs first, the state behind it ----
+    long u;
+    {
+        const int ee = (int)ev;
+        u = unique_index<P>(ee % a.nx, (ee / a.nx) % a.ny, ee / (a.nx * a.ny), i, j, k, a.nx, a.ny);
+    }
+    load_tables<P, EPB, NT>(a, tile, cf, &gtab[0][0]);
+    if (t < EPB) {
+        const int se = tile * EPB + t;
+        if (a.src_slot)
+            lds_load_dword((const int *)a.src_slot + (se < a.nel ? se : a.nel - 1), lds_address(sst));
+        else
+            sst[t] = -1;
+    }
+    int soff = 0, moff = 0;   // LDS places of the tile's first words
+    R v[3], sg[6], lo[6], M[!DMA && VISCO ? NM : 1], lam, mu, tau = R(0);
+    const int ne = a.nel - tile * EPB < EPB ? a.nel - tile * EPB : EPB;   // elements of the tile
+    if constexpr (DMA) {
+        const int w = t & ~63;
+        lds_load_dword((const R *)a.vx + u, lds_address(vbuf + w));
+        lds_load_dword((const R *)a.vy + u, lds_address(vbuf + NT + w));
+        lds_load_dword((const R *)a.vz + u, lds_address(vbuf + 2 * NT + w));
+        soff = lds_load_run<TW, NT>((const float *)a.sig, (long)tile * TW, ne * NS * NP, sbuf);
+        if constexpr (MAT) moff = lds_load_run<MW, NT>((const float *)a.lam, (long)tile * MW, ne * NC * NP, mbuf);
+        if constexpr (S16) {
+            const long mb = em_index(ev, NC, 0, NP, node);
+            lam = (R)(float)a.s16.lam[mb];
+            mu = (R)(float)a.s16.mu[mb];
+            if constexpr (VISCO) tau = (R)(float)a.s16.tau[mb];
+        }
+    } else {
+        v[0] = a.vx[u];
+        v[1] = a.vy[u];
+        v[2] = a.vz[u];
 #pragma unroll
-        for (int c = 0; c < NM; ++c)
-            lds_dma_dword(mem + c * NP, base + (unsigned)(c * S::NT * sizeof(R)));
+        for (int c = 0; c < 6; ++c) sg[c] = a.sig[em_index(ev, NS, c, NP, node)];
+        const long mb = em_index(ev, NC, 0, NP, node);
+        lam = a.lam[mb];
+        mu = a.mu[mb];
+        if constexpr (VISCO) tau = a.tau[mb];
+#pragma unroll
+        for (int c = 0; c < NM; ++c) M[c] = a.mem[em_index(ev, NS, c, NP, node)];
     }
-
-    // ---- tables of the tile: every lane loads from clamped (in-bounds)
-    // indices, the lanes owning an entry store it after the state loads are
-    // issued, so table and state loads share one round trip ----
-    static_assert(P1 * P1 <= S::NT, "coefficient fill needs (p+1)^2 lanes");
-    static_assert(NE * P1 <= S::NT, "one geometry entry per lane");
-    const int tq = t < P1 * P1 ? t : 0;
-    const C tD0 = a.Dx[tq], tD1 = a.Dy[tq], tD2 = a.Dz[tq], tD3 = a.dlw[tq];
-    const C tW = a.w[t < P1 ? t : 0];
-    const int xg = t < NE * P1 ? t : 0;
-    const int ges = xg / P1, gq = xg - ges * P1;
-    int ge = tile0 * EPB + ges;
-    ge = ge < a.nel ? ge : a.nel - 1;
-    const int gex = ge % a.nx, gey = (ge / a.nx) % a.ny, gez = ge / (a.nx * a.ny);
-    const ThTab<C> th = a.tth[gex * P1 + gq];
-    const RTab<C> rr = a.tr[gez * P1 + gq];
-    // the profiles exist (zero) also without a taper
-    const double gpx = a.px[gex * P1 + gq], gpy = a.py[gey * P1 + gq], gpz = a.pz[gez * P1 + gq];
-    const int se = tile0 * EPB + (t < NE ? t : 0);
-    int sslot = -1;
-    if (a.src_slot) sslot = a.src_slot[se < a.nel ? se : a.nel - 1];
-
-    // ---- state of the tile ----
-    TileState<R, VM> cur;
-    load_tile<P, E, R, VM, S16, !MDMA, KS>(a, tile0, cur);
-
-    if (t < P1 * P1) {
-        cf[0][t] = tD0;
-        cf[1][t] = tD1;
-        cf[2][t] = tD2;
-        cf[3][t] = tD3;
-    }
-    if (t < P1) cw[t] = tW;
-    if (t < NE * P1) {
-        C *g = gtab[ges];
-        g[G_SIN * P1 + gq] = th.sin_t;
-        g[G_ISIN * P1 + gq] = th.inv_sin;
-        g[G_COT * P1 + gq] = th.cot;
-        g[G_R * P1 + gq] = rr.r;
-        g[G_IR * P1 + gq] = rr.inv_r;
-        g[G_R2 * P1 + gq] = rr.r2;
-        g[G_PX * P1 + gq] = a.taper_on ? (C)gpx : C(0);
-        g[G_PY * P1 + gq] = a.taper_on ? (C)gpy : C(0);
-        g[G_PZ * P1 + gq] = a.taper_on ? (C)gpz : C(0);
-    }
-    if (t < NE) sst[t] = se < a.nel ? sslot : -1;
     // iteration it = *it_dev + 1 uses the STF sample it-1 (zero for it = 1)
     const int it = *a.it_dev + 1;
 
+    const C *gs = gtab[es];
+
+    // LDS views: velocity component c of node n of this lane's element at
+    // lv[c * VS + n], effective stress component c at ls[c * SS + n] (FP32: the
+    // state block's component c)
+    constexpr int VS = DMA ? NT : EPB * NP, SS = DMA ? NP : EPB * NP;
+    R *const lv = (DMA ? vbuf : sbuf) + es * NP;
+    R *const ls = DMA ? sbuf + soff + es * (NS * NP) : lv;
+    const R *const lm = mbuf + moff + es * (NC * NP) + node;
+    if constexpr (DMA) {
+        // tables and velocity: all but the state's loads, which only a whole
+        // tile issues in full
+        if (ne == EPB)
+            wait_loads<run_loads(TW, NT) + (MAT ? run_loads(MW, NT) : 0)>();
+        else
+            wait_loads<0>();
+    } else if (inside) {
+        // the tables' loads are older than those of v
+#pragma unroll
+        for (int c = 0; c < 3; ++c) lv[c * VS + node] = v[c];
+        asm volatile("" ::: "memory");
+    }
+    __syncthreads();
+
+    // ---- K1: tensor-product derivatives along theta, phi, r ----
+    C dxv[3] = {0, 0, 0}, dyv[3] = {0, 0, 0}, dzv[3] = {0, 0, 0};
     {
-        const int tile = tile0;
-        const int es = inside ? slot : 0;
-        const int e = tile * EPB + slot;
-        const bool valid = inside && e < a.nel;
-        const long eb = (long)(valid ? e : 0) * NP + node;    // element-local address
-        const long ev = valid ? e : 0;
-        const C *gs = gtab[es];
+        const C *Dxi = cf + i * P1;
+        const C *Dyj = cf + P1 * P1 + j * P1;
+        const C *Dzk = cf + 2 * P1 * P1 + k * P1;
+#pragma unroll
+        for (int q = 0; q < P1; ++q) {
+            const R *vx = lv + q + P1 * (j + P1 * k);
+            const R *vy = lv + i + P1 * (q + P1 * k);
+            const R *vz = lv + i + P1 * (j + P1 * q);
+            const C cx = Dxi[q], cy = Dyj[q], cz = Dzk[q];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                dxv[c] += (C)vx[c * VS] * cx;
+                dyv[c] += (C)vy[c * VS] * cy;
+                dzv[c] += (C)vz[c * VS] * cz;
+            }
+        }
+    }
 
-        if (inside) lds.put_v(L + node, cur.v[0], cur.v[1], cur.v[2]);
-        // tables and velocity in LDS
+    // ---- K2: spherical completion, K4: symmetrisation ----
+    R exx, eyy, ezz, exy, exz, eyz;
+    {
+        const C ux = DMA ? lv[node] : v[0], uy = DMA ? lv[VS + node] : v[1], uz = DMA ? lv[2 * VS + node] : v[2];
+        const C inv_r = gs[G_IR * P1 + k];
+        const C cot = gs[G_COT * P1 + i];
+        const C inv_rs = inv_r * gs[G_ISIN * P1 + i];
+        const C ezx = -dzv[0];
+        const C exz_c = (dxv[2] - ux) * inv_r;
+        const C ezy = -dzv[1];
+        const C eyz_c = -uy * inv_r + dyv[2] * inv_rs;
+        const C exy_c = dxv[1] * inv_r;
+        const C eyx = -uy * cot * inv_r + dyv[0] * inv_rs;
+        const C gxx = (uz + dxv[0]) * inv_r;
+        const C gyy = dyv[1] * inv_rs + (uz + ux * cot) * inv_r;
+        const C gzz = -dzv[2];
+        const C gxy = (exy_c + eyx) * 0.5;
+        const C gxz = (exz_c + ezx) * 0.5;
+        const C gyz = (eyz_c + ezy) * 0.5;
+        exx = (R)gxx;
+        eyy = (R)gyy;
+        ezz = (R)gzz;
+        exy = (R)gxy;
+        exz = (R)gxz;
+        eyz = (R)gyz;
+        // K3: the displacement gradient integrates the velocity gradient
+        // (src/evolution.f90:179-187); kept as its symmetric part, the
+        // only form the reference outputs (src/volume_snapshot.f90:220-236),
+        // in FP64, and only when requested
+        if (a.dgrad && valid) {
+            double *g = a.dgrad + em_index(ev, 6, 0, NP, node);
+            g[0 * NP] += a.dt * (double)gxx;
+            g[1 * NP] += a.dt * (double)gxy;
+            g[2 * NP] += a.dt * (double)gxz;
+            g[3 * NP] += a.dt * (double)gyy;
+            g[4 * NP] += a.dt * (double)gyz;
+            g[5 * NP] += a.dt * (double)gzz;
+        }
+    }
+
+    if constexpr (DMA) {
+        // the state, of every wave
+        wait_loads<0>();
         __syncthreads();
+    }
+    // memory variable c of this lane's node, as the step found it
+    auto mem = [&](int c) -> R { return DMA ? ls[(NS - NM + c) * NP + node] : M[c]; };
+    if constexpr (MAT) {
+        lam = lm[0];
+        mu = lm[NP];
+        if constexpr (VISCO) tau = lm[2 * NP];
+    }
 
-        // ---- K1: tensor-product derivatives along theta, phi, r ----
-        C dxv[3] = {0, 0, 0}, dyv[3] = {0, 0, 0}, dzv[3] = {0, 0, 0};
-        {
-            const C *Dxi = cf[0] + i * P1;
-            const C *Dyj = cf[1] + j * P1;
-            const C *Dzk = cf[2] + k * P1;
+    // ---- K5: stress rate times dt (lam, mu, A, B, C carry the dt) ----
+    R rt[6];
+    const R tmu = R(2) * mu;
+    if constexpr (!VISCO) {
+        const R Lr = lam * (exx + eyy + ezz);
+        rt[XX] = Lr + tmu * exx;
+        rt[YY] = Lr + tmu * eyy;
+        rt[ZZ] = Lr + tmu * ezz;
+        rt[XY] = tmu * exy;
+        rt[XZ] = tmu * exz;
+        rt[YZ] = tmu * eyz;
+    } else {
+        // SLS in the loop form of the commented-out src/evolution.f90:216-284:
+        // lam holds kappa - 2 mu_tau / 3 and mu holds mu_tau = mu (1 + tau),
+        // both formed in FP64; 2 mu itself only scales the memory variables
+        const R tmut = tmu;                                    // 2 mu_tau
+        const R tm = tmut / (R(1) + tau);                      // 2 mu
+        if constexpr (VM == 6) {
+            R Md[6];
 #pragma unroll
-            for (int q = 0; q < P1; ++q) {
-                const int nxq = L + q + P1 * (j + P1 * k);
-                const int nyq = L + i + P1 * (q + P1 * k);
-                const int nzq = L + i + P1 * (j + P1 * q);
-                const C cx = Dxi[q], cy = Dyj[q], cz = Dzk[q];
-                R vx[3], vy[3], vz[3];
-                lds.get_v(nxq, vx);
-                lds.get_v(nyq, vy);
-                lds.get_v(nzq, vz);
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    dxv[c] += (C)vx[c] * cx;
-                    dyv[c] += (C)vy[c] * cy;
-                    dzv[c] += (C)vz[c] * cz;
-                }
-            }
-        }
-
-        // ---- K2: spherical completion, K4: symmetrisation ----
-        R exx, eyy, ezz, exy, exz, eyz;
-        {
-            const C ux = cur.v[0], uy = cur.v[1], uz = cur.v[2];
-            const C inv_r = gs[G_IR * P1 + k];
-            const C cot = gs[G_COT * P1 + i];
-            const C inv_rs = inv_r * gs[G_ISIN * P1 + i];
-            const C ezx = -dzv[0];
-            const C exz_c = (dxv[2] - ux) * inv_r;
-            const C ezy = -dzv[1];
-            const C eyz_c = -uy * inv_r + dyv[2] * inv_rs;
-            const C exy_c = dxv[1] * inv_r;
-            const C eyx = -uy * cot * inv_r + dyv[0] * inv_rs;
-            const C gxx = (uz + dxv[0]) * inv_r;
-            const C gyy = dyv[1] * inv_rs + (uz + ux * cot) * inv_r;
-            const C gzz = -dzv[2];
-            const C gxy = (exy_c + eyx) * 0.5;
-            const C gxz = (exz_c + ezx) * 0.5;
-            const C gyz = (eyz_c + ezy) * 0.5;
-            exx = (R)gxx;
-            eyy = (R)gyy;
-            ezz = (R)gzz;
-            exy = (R)gxy;
-            exz = (R)gxz;
-            eyz = (R)gyz;
-            // K3: the displacement gradient integrates the velocity gradient
-            // (src/evolution.f90:179-187); kept as its symmetric part, the
-            // only form the reference outputs (src/volume_snapshot.f90:220-236),
-            // in FP64, and only when requested
-            if (a.dgrad && valid) {
-                double *g = a.dgrad + em_index(ev, 6, 0, NP, node);
-                g[0 * NP] += a.dt * (double)gxx;
-                g[1 * NP] += a.dt * (double)gxy;
-                g[2 * NP] += a.dt * (double)gxz;
-                g[3 * NP] += a.dt * (double)gyy;
-                g[4 * NP] += a.dt * (double)gyz;
-                g[5 * NP] += a.dt * (double)gzz;
-            }
-        }
-
-        // ---- K5: stress rate times dt (lam, mu, A, B, C carry the dt) ----
-        R rt[6];
-        const R tmu = R(2) * cur.mu;
-        if constexpr (!VISCO) {
-            const R Lr = cur.lam * (exx + eyy + ezz);
-            rt[XX] = Lr + tmu * exx;
-            rt[YY] = Lr + tmu * eyy;
-            rt[ZZ] = Lr + tmu * ezz;
-            rt[XY] = tmu * exy;
-            rt[XZ] = tmu * exz;
-            rt[YZ] = tmu * eyz;
+            for (int c = 0; c < 6; ++c) Md[c] = mem(c) + mem(6 + c) + mem(12 + c);
+            const R Msum = Md[XX] + Md[YY] + Md[ZZ];
+            const R Lr = lam * (exx + eyy + ezz) - tm * Msum * R(1.0 / 3.0);
+            rt[XX] = Lr + tmut * exx + tm * Md[XX];
+            rt[YY] = Lr + tmut * eyy + tm * Md[YY];
+            rt[ZZ] = Lr + tmut * ezz + tm * Md[ZZ];
+            rt[XY] = tmut * exy + tm * Md[XY];
+            rt[XZ] = tmut * exz + tm * Md[XZ];
+            rt[YZ] = tmut * eyz + tm * Md[YZ];
         } else {
-            // SLS in the loop form of the commented-out src/evolution.f90:216-284
-            if constexpr (MDMA) {
-                // this lane's words were written by its own wave's loads
-                const int z = wait_vmem_zero();
+            // The memory variables enter the stress rate only as
+            // Md - tr(Md)/3 I, and every component relaxes at the same
+            // rate with the same forcing (t3 e), so their deviatoric
+            // part evolves on its own, driven by the deviatoric strain
+            // rate: five words per mechanism hold it (xx xy xz yy yz,
+            // zz = -(xx + yy)), and the trace is never formed.
+            R Dd[5];
 #pragma unroll
-                for (int c = 0; c < NM; ++c) cur.M[c] = mbuf[c][t + z];
-            }
-            // lam holds kappa - 2 mu_tau / 3 and mu holds mu_tau = mu (1 + tau),
-            // both formed in FP64; 2 mu itself only scales the memory variables
-            const R tmut = tmu;                                    // 2 mu_tau
-            const R tm = tmut / (R(1) + cur.tau);                  // 2 mu
-            if constexpr (VM == 6) {
-                R Md[6];
-#pragma unroll
-                for (int c = 0; c < 6; ++c) Md[c] = cur.M[c] + cur.M[6 + c] + cur.M[12 + c];
-                const R Msum = Md[XX] + Md[YY] + Md[ZZ];
-                const R Lr = cur.lam * (exx + eyy + ezz) - tm * Msum * R(1.0 / 3.0);
-                rt[XX] = Lr + tmut * exx + tm * Md[XX];
-                rt[YY] = Lr + tmut * eyy + tm * Md[YY];
-                rt[ZZ] = Lr + tmut * ezz + tm * Md[ZZ];
-                rt[XY] = tmut * exy + tm * Md[XY];
-                rt[XZ] = tmut * exz + tm * Md[XZ];
-                rt[YZ] = tmut * eyz + tm * Md[YZ];
-            } else {
-                // The memory variables enter the stress rate only as
-                // Md - tr(Md)/3 I, and every component relaxes at the same
-                // rate with the same forcing (t3 e), so their deviatoric
-                // part evolves on its own, driven by the deviatoric strain
-                // rate: five words per mechanism hold it (xx xy xz yy yz,
-                // zz = -(xx + yy)), and the trace is never formed.
-                R Dd[5];
-#pragma unroll
-                for (int c = 0; c < 5; ++c) Dd[c] = cur.M[c] + cur.M[5 + c] + cur.M[10 + c];
-                const R Dzz = -(Dd[XX] + Dd[YY]);
-                const R Lr = cur.lam * (exx + eyy + ezz);
-                rt[XX] = Lr + tmut * exx + tm * Dd[XX];
-                rt[YY] = Lr + tmut * eyy + tm * Dd[YY];
-                rt[ZZ] = Lr + tmut * ezz + tm * Dzz;
-                rt[XY] = tmut * exy + tm * Dd[XY];
-                rt[XZ] = tmut * exz + tm * Dd[XZ];
-                rt[YZ] = tmut * eyz + tm * Dd[YZ];
-            }
+            for (int c = 0; c < 5; ++c) Dd[c] = mem(c) + mem(5 + c) + mem(10 + c);
+            const R Dzz = -(Dd[XX] + Dd[YY]);
+            const R Lr = lam * (exx + eyy + ezz);
+            rt[XX] = Lr + tmut * exx + tm * Dd[XX];
+            rt[YY] = Lr + tmut * eyy + tm * Dd[YY];
+            rt[ZZ] = Lr + tmut * ezz + tm * Dzz;
+            rt[XY] = tmut * exy + tm * Dd[XY];
+            rt[XZ] = tmut * exz + tm * Dd[XZ];
+            rt[YZ] = tmut * eyz + tm * Dd[YZ];
         }
-        if (S16 ? a.s16.ca != nullptr : a.ca != nullptr) {   // anisotropy (src/evolution.f90:290-296)
-            R pa, pb, pc;
-            if constexpr (S16) {
-                pa = (R)(float)a.s16.ca[eb];
-                pb = (R)(float)a.s16.cb[eb];
-                pc = (R)(float)a.s16.cc[eb];
-            } else {
-                pa = a.ca[eb];
-                pb = a.cb[eb];
-                pc = a.cc[eb];
-            }
-            rt[XX] += pc * ezz + pa * (eyy + exx);
-            rt[YY] += pc * ezz + pa * (eyy + exx);
-            rt[ZZ] += pc * (eyy + exx);
-            rt[XZ] += R(2) * pb * exz;
-            rt[YZ] += R(2) * pb * eyz;
+    }
+    if (S16 ? a.s16.ca != nullptr : a.ca != nullptr) {   // anisotropy (src/evolution.f90:290-296)
+        R pa, pb, pc;
+        if constexpr (S16) {
+            pa = (R)(float)a.s16.ca[eb];
+            pb = (R)(float)a.s16.cb[eb];
+            pc = (R)(float)a.s16.cc[eb];
+        } else {
+            pa = a.ca[eb];
+            pb = a.cb[eb];
+            pc = a.cc[eb];
         }
+        rt[XX] += pc * ezz + pa * (eyy + exx);
+        rt[YY] += pc * ezz + pa * (eyy + exx);
+        rt[ZZ] += pc * (eyy + exx);
+        rt[XZ] += R(2) * pb * exz;
+        rt[YZ] += R(2) * pb * eyz;
+    }
 
-        // ---- K6: integrate the stress ----
-        R sg[6], lo[6];
+    // ---- K6: integrate the stress ----
+    if constexpr (DMA) {
+#pragma unroll
+        for (int c = 0; c < 6; ++c) sg[c] = ls[c * NP + node];
+    }
+    if constexpr (KS == 1) {
+#pragma unroll
+        for (int c = 0; c < 6; ++c) lo[c] = ls[(6 + c) * NP + node];
+    } else if constexpr (KS == 2) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const unsigned w = __builtin_bit_cast(unsigned, (float)ls[(6 + q) * NP + node]);
+            lo[2 * q] = (R)bf16_lo(w);
+            lo[2 * q + 1] = (R)bf16_hi(w);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+        if constexpr (KS != 0)
+            kahan_add(sg[c], lo[c], rt[c]);
+        else
+            sg[c] = sg[c] + rt[c];
+    }
+
+    // ---- K7: moment-tensor glut and single force of the previous add() ----
+    R src[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    const int sl = sst[es];
+    if (valid && sl >= 0 && it > 1 && it <= a.nt) {
+#pragma unroll
+        for (int c = 0; c < 9; ++c) {
+            const int ch = a.src_chan[sl * 9 + c];
+            if (ch >= 0) {
+                const double d = a.stf[(long)ch * a.nt + (it - 2)];
+                src[c] = (R)(-(d * a.src_coef[((long)sl * 9 + c) * NP + node]));
+            }
+        }
+    }
+
+    if constexpr (!DMA) __syncthreads();   // the staged velocity is no longer needed
+    if (inside) {
+        // effective stress, with the glut
+#pragma unroll
+        for (int c = 0; c < 6; ++c) ls[c * SS + node] = sg[c] + src[c];
+    }
+
+    // ---- taper factor of this node (K13) ----
+    R dmp = R(0);   // 1 - taper
+    {
+        const C tx = gs[G_PX * P1 + i], ty = gs[G_PY * P1 + j], tz = gs[G_PZ * P1 + k];
+        if (tx + ty + tz != C(0)) dmp = (R)taper_damp(tx, ty, tz, a.alpha);
+    }
+
+    // ---- tapered stress (K13) and its compensation ----
+    unsigned lo2[3];
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+        sg[c] = sg[c] - sg[c] * dmp;
+        if constexpr (KS != 0) lo[c] = lo[c] - lo[c] * dmp;
+    }
+    if constexpr (KS == 2) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) lo2[q] = pack_bf16((float)lo[2 * q], (float)lo[2 * q + 1]);
+    }
+
+    // ---- store them and the new memory variables (loop form of
+    // src/evolution.f90:415-442) ----
+    auto store_state = [&]() {
 #pragma unroll
         for (int c = 0; c < 6; ++c) {
-            sg[c] = cur.sg[c];
-            lo[c] = cur.lo[c];
+            a.sig_w[em_index(ev, NS, c, NP, node)] = sg[c];
+            if constexpr (KS == 1) a.sig_lo_w[em_index(ev, NS, c, NP, node)] = lo[c];
         }
-        if constexpr (KS != 0) {
-            if constexpr (KS == 2) {
+        if constexpr (KS == 2) {
 #pragma unroll
-                for (int q = 0; q < 3; ++q) {
-                    lo[2 * q] = (R)bf16_lo(cur.lo2[q]);
-                    lo[2 * q + 1] = (R)bf16_hi(cur.lo2[q]);
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < 6; ++c) kahan_add(sg[c], lo[c], rt[c]);
-        } else {
-#pragma unroll
-            for (int c = 0; c < 6; ++c) sg[c] = sg[c] + rt[c];
+            for (int q = 0; q < 3; ++q) a.sig_lo2_w[em_index(ev, NS, q, NP, node)] = lo2[q];
         }
-
-        // ---- K7: moment-tensor glut and single force of the previous add() ----
-        R src[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-        const int sslot = sst[es];
-        if (valid && sslot >= 0 && it > 1 && it <= a.nt) {
-#pragma unroll
-            for (int c = 0; c < 9; ++c) {
-                const int ch = a.src_chan[sslot * 9 + c];
-                if (ch >= 0) {
-                    const double d = a.stf[(long)ch * a.nt + (it - 2)];
-                    src[c] = (R)(-(d * a.src_coef[((long)sslot * 9 + c) * NP + node]));
-                }
-            }
-        }
-
-        __syncthreads();   // LDS velocity no longer needed
-        if (inside) {
-            R se[6];   // effective stress, with the glut
-#pragma unroll
-            for (int c = 0; c < 6; ++c) se[c] = sg[c] + src[c];
-            lds.put_s(L + node, se);
-        }
-
-        // ---- memory variables (loop form of src/evolution.f90:415-442) ----
-        R M[VISCO ? NM : 1];
         if constexpr (VISCO) {
             // M (1 - dt/tau_p) - dt tau / (3 tau_p) e  ==  M - dt/tau_p (M + tau/3 e):
             // the decrement form keeps the FP32 relaxation rate exact to one
             // rounding of dt/tau_p (1 - dt/tau_p would lose its low bits)
-            const R t3 = cur.tau * R(1.0 / 3.0);
-            R ev[6] = {exx, exy, exz, eyy, eyz, ezz};
+            const R t3 = tau * R(1.0 / 3.0);
+            R em[6] = {exx, exy, exz, eyy, eyz, ezz};
             if constexpr (VM == 5) {   // deviatoric strain rate
                 const R tr3 = (exx + eyy + ezz) * R(1.0 / 3.0);
-                ev[XX] = exx - tr3;
-                ev[YY] = eyy - tr3;
+                em[XX] = exx - tr3;
+                em[YY] = eyy - tr3;
             }
 #pragma unroll
             for (int m = 0; m < NRDISS; ++m) {
 #pragma unroll
-                for (int c = 0; c < VM; ++c)
-                    M[VM * m + c] = cur.M[VM * m + c] - a.rate[m] * (cur.M[VM * m + c] + t3 * ev[c]);
-            }
-        }
-
-        // ---- taper factor of this node (K13) ----
-        R dmp = R(0);   // 1 - taper
-        {
-            const C tx = gs[G_PX * P1 + i], ty = gs[G_PY * P1 + j], tz = gs[G_PZ * P1 + k];
-            if (tx + ty + tz != C(0)) dmp = (R)taper_damp(tx, ty, tz, a.alpha);
-        }
-
-        // ---- store tapered stress (K13) and memory variables ----
-        auto store_state = [&]() {
-            if constexpr (KS == 1) {
-#pragma unroll
-                for (int c = 0; c < 6; ++c) {
-                    a.sig_w[em_index(ev, NS, c, NP, node)] = sg[c] - sg[c] * dmp;
-                    a.sig_lo_w[em_index(ev, NS, c, NP, node)] = lo[c] - lo[c] * dmp;
+                for (int c = 0; c < VM; ++c) {
+                    const R x = mem(VM * m + c);
+                    a.mem_w[em_index(ev, NS, VM * m + c, NP, node)] = x - a.rate[m] * (x + t3 * em[c]);
                 }
-            } else if constexpr (KS == 2) {
-#pragma unroll
-                for (int c = 0; c < 6; ++c) a.sig_w[em_index(ev, NS, c, NP, node)] = sg[c] - sg[c] * dmp;
-#pragma unroll
-                for (int q = 0; q < 3; ++q)
-                    a.sig_lo2_w[em_index(ev, NS, q, NP, node)] = pack_bf16((float)(lo[2 * q] - lo[2 * q] * dmp),
-                                                       (float)(lo[2 * q + 1] - lo[2 * q + 1] * dmp));
-            } else {
-#pragma unroll
-                for (int c = 0; c < 6; ++c) a.sig_w[em_index(ev, NS, c, NP, node)] = sg[c] - sg[c] * dmp;
-            }
-            if constexpr (VISCO) {
-#pragma unroll
-                for (int c = 0; c < NM; ++c) a.mem_w[em_index(ev, NS, c, NP, node)] = M[c];
-            }
-        };
-        if constexpr (EARLY) {
-            if (valid) store_state();
-        }
-
-        __syncthreads();
-
-        // ---- K8: weak divergence ----
-        C ax[P1], ay[P1], az[P1];
-        {
-            const C *dli = cf[3] + i * P1;
-            const C *dlj = cf[3] + j * P1;
-            const C *dlk = cf[3] + k * P1;
-#pragma unroll
-            for (int q = 0; q < P1; ++q) {
-                ax[q] = dli[q] * gs[G_SIN * P1 + q];
-                ay[q] = dlj[q];
-                az[q] = dlk[q] * gs[G_R2 * P1 + q];
             }
         }
-        C Sx[3] = {0, 0, 0}, Sy[3] = {0, 0, 0}, Sz[3] = {0, 0, 0};
+    };
+    if constexpr (EARLY) {
+        if (valid) store_state();
+    }
+
+    __syncthreads();
+
+    // ---- K8: weak divergence ----
+    C Sx[3] = {0, 0, 0}, Sy[3] = {0, 0, 0}, Sz[3] = {0, 0, 0};
+    {
+        const C *dl = cf + 3 * P1 * P1;
+        const C *dli = dl + i * P1, *dlj = dl + j * P1, *dlk = dl + k * P1;
+        // x contraction: sxx, sxy, sxz feed sx, sy, sz; y: sxy, syy, syz;
+        // z: sxz, syz, szz
+        constexpr int comp[3][3] = {{XX, XY, XZ}, {XY, YY, YZ}, {XZ, YZ, ZZ}};
 #pragma unroll
         for (int q = 0; q < P1; ++q) {
-            const int nxq = L + q + P1 * (j + P1 * k);
-            const int nyq = L + i + P1 * (q + P1 * k);
-            const int nzq = L + i + P1 * (j + P1 * q);
-            // x contraction: sxx, sxy, sxz feed sx, sy, sz; y: sxy, syy,
-            // syz; z: sxz, syz, szz
-            R wx[3], wy[3], wz[3];
-            lds.get_s(0, nxq, wx);
-            lds.get_s(1, nyq, wy);
-            lds.get_s(2, nzq, wz);
+            const R *wx = ls + q + P1 * (j + P1 * k);
+            const R *wy = ls + i + P1 * (q + P1 * k);
+            const R *wz = ls + i + P1 * (j + P1 * q);
+            const C ax = dli[q] * gs[G_SIN * P1 + q], ay = dlj[q], az = dlk[q] * gs[G_R2 * P1 + q];
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
-                Sx[c] += ax[q] * (C)wx[c];
-                Sy[c] += ay[q] * (C)wy[c];
-                Sz[c] += az[q] * (C)wz[c];
+                Sx[c] += ax * (C)wx[comp[0][c] * SS];
+                Sy[c] += ay * (C)wy[comp[1][c] * SS];
+                Sz[c] += az * (C)wz[comp[2][c] * SS];
             }
         }
-        const C rk = gs[G_R * P1 + k];
-        const C Cx = cw[j] * cw[k] * rk * a.d1;
-        const C Cy = cw[i] * cw[k] * rk * a.d2;
-        const C Cz = cw[i] * cw[j] * gs[G_SIN * P1 + i] * a.d3;
+    }
+    const C rk = gs[G_R * P1 + k];
+    const C *cw = cf + 4 * P1 * P1;
+    const C Cx = cw[j] * cw[k] * rk * a.d1;
+    const C Cy = cw[i] * cw[k] * rk * a.d2;
+    const C Cz = cw[i] * cw[j] * gs[G_SIN * P1 + i] * a.d3;
 
-        if (valid) {
+    if (valid) {
 #pragma unroll
-            for (int c = 0; c < 3; ++c)
-                a.force[force_index<P>(ev, c, node, a.nel)] = (R)((C)src[6 + c] + Cz * Sz[c] + Cy * Sy[c] + Cx * Sx[c]);
-
-            if constexpr (!EARLY) store_state();
-        }
+        for (int c = 0; c < 3; ++c)
+            a.force[force_index<P>(ev, c, node, a.nel)] = (R)((C)src[6 + c] + Cz * Sz[c] + Cy * Sy[c] + Cx * Sx[c]);
+        if constexpr (!EARLY) store_state();
     }
 }
 
@@ -796,8 +770,17 @@ __host__ __device__ inline int record_blocks(int receivers, int lanes)
     return ((receivers + per - 1) / per + 7) / 8 * 8;
 }
 
-template <int P, int E, typename R, int VM, bool S16, int KS, int LL>
-__global__ void __launch_bounds__((Shape<P, E>::NT))
+// Waves per SIMD that the registers must leave room for: one-element FP32
+// workgroups of order 6 have 6 waves, and 3 of them fit a CU only at 5 waves
+// per SIMD (96 VGPRs; with stress compensation they take 101 to 103 by
+// themselves and ran 525 us at 40x36x20 with 2 workgroups per CU, 483 us with
+// 3), those of order 7 have 8 waves, and 2 fit at 4 (128 VGPRs; one variant
+// took 130: 566 us at 36x30x18 against 453).
+template <int P, int E, typename R>
+constexpr int min_waves() { return sizeof(R) == 4 && Shape<P, E>::EPB == 1 ? (P == 6 ? 5 : P == 7 ? 4 : 1) : 1; }
+
+template <int P, int E, typename R, int VM, bool S16, int KS>
+__global__ void __launch_bounds__((Shape<P, E>::NT), (min_waves<P, E, R>()))
 elem_kernel(const ElemArgs<R> a, const RecArgs<R> rec)
 {
     constexpr int NT = Shape<P, E>::NT;
@@ -807,11 +790,11 @@ elem_kernel(const ElemArgs<R> a, const RecArgs<R> rec)
         if (r < rec.n) record_body<P, R, false>(rec, r);
         return;
     }
-    elem_body<P, E, R, VM, S16, KS, LL>(a, chunk_block(b, gridDim.x - nb, a.remap));
+    elem_body<P, E, R, VM, S16, KS>(a, chunk_block(b, gridDim.x - nb, a.remap));
 }
 
-template <int P, int E, typename R, int VM, int KS, int LL>
-__global__ void __launch_bounds__((Shape<P, E>::NT))
+template <int P, int E, typename R, int VM, int KS>
+__global__ void __launch_bounds__((Shape<P, E>::NT), (min_waves<P, E, R>()))
 elem_kernel_batch(const ElemArgs<R> *__restrict__ args, const int2 *__restrict__ own,
                   const RecArgs<R> *__restrict__ recs, const int2 *__restrict__ rown, int nrec)
 {
@@ -825,7 +808,7 @@ elem_kernel_batch(const ElemArgs<R> *__restrict__ args, const int2 *__restrict__
     // (simulation, its workgroup index), in XCD-aware order over the whole
     // batch
     const int2 o = own[chunk_block(b, gridDim.x - nb, 1)];
-    elem_body<P, E, R, VM, false, KS, LL>(args[o.x], o.y);
+    elem_body<P, E, R, VM, false, KS>(args[o.x], o.y);
 }
 
 }  // namespace s3d

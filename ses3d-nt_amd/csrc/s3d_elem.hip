@@ -2,7 +2,7 @@
 // Compiled once per order (2..7) so that the orders' instantiations of
 // elem_kernel / elem_kernel_batch build in parallel. A launch description
 // (s3d_launch.h) selects the instantiation: element tile, memory words per
-// mechanism, stress compensation, kernel variant, BF16 statics. The choices
+// mechanism, stress compensation, BF16 statics. The choices
 // are template parameters so that no run-time branch inside the kernel
 // leaves register joins that wait for every load in flight.
 #include "s3d_elem.h"
@@ -20,33 +20,22 @@ namespace {
 template <int P, int E>
 unsigned tiles(long nel) { return (unsigned)((nel + Shape<P, E>::EPB - 1) / Shape<P, E>::EPB); }
 
-// stress compensation (FP32 only)
-template <int P, int E, typename R, int VM, bool S16, int LL>
-void launch_ks(int ks, const ElemArgs<R> &ea, const RecArgs<R> &ra, hipStream_t st, unsigned ge)
+template <int P, int E, typename R, int VM, bool S16, int KS>
+void launch(const ElemArgs<R> &ea, const RecArgs<R> &ra, hipStream_t st, unsigned ge)
 {
-    constexpr int NT = Shape<P, E>::NT;
-    if (ks == 1)
-        hipLaunchKernelGGL((elem_kernel<P, E, R, VM, S16, 1, LL>), dim3(ge), dim3(NT), 0, st, ea, ra);
-    else if (ks == 2)
-        hipLaunchKernelGGL((elem_kernel<P, E, R, VM, S16, 2, LL>), dim3(ge), dim3(NT), 0, st, ea, ra);
-    else
-        hipLaunchKernelGGL((elem_kernel<P, E, R, VM, S16, 0, LL>), dim3(ge), dim3(NT), 0, st, ea, ra);
+    hipLaunchKernelGGL((elem_kernel<P, E, R, VM, S16, KS>), dim3(ge), dim3(Shape<P, E>::NT),
+                       (spare_lds<P, E, R, VM, S16, KS>()), st, ea, ra);
 }
 
-// kernel variant and stress compensation: FP32 only; FP64 and the
-// BF16-static kernels use variant 0 without compensation words
+// stress compensation: FP32 only
 template <int P, int E, typename R, int VM, bool S16>
-void launch_ll(int ks, int ll, const ElemArgs<R> &ea, const RecArgs<R> &ra, hipStream_t st, unsigned ge)
+void launch_ks(int ks, const ElemArgs<R> &ea, const RecArgs<R> &ra, hipStream_t st, unsigned ge)
 {
     if constexpr (std::is_same<R, float>::value) {
-        if constexpr (!S16) {
-            if (ll == 1) return launch_ks<P, E, R, VM, S16, 1>(ks, ea, ra, st, ge);
-            if (ll == 2) return launch_ks<P, E, R, VM, S16, 2>(ks, ea, ra, st, ge);
-        }
-        launch_ks<P, E, R, VM, S16, 0>(ks, ea, ra, st, ge);
-    } else {
-        hipLaunchKernelGGL((elem_kernel<P, E, R, VM, S16, 0, 0>), dim3(ge), dim3(Shape<P, E>::NT), 0, st, ea, ra);
+        if (ks == 1) return launch<P, E, R, VM, S16, 1>(ea, ra, st, ge);
+        if (ks == 2) return launch<P, E, R, VM, S16, 2>(ea, ra, st, ge);
     }
+    launch<P, E, R, VM, S16, 0>(ea, ra, st, ge);
 }
 
 template <int P, int E, typename R>
@@ -55,47 +44,33 @@ void launch_vm(const ElemLaunch &l, const ElemArgs<R> &ea, const RecArgs<R> &ra,
     const unsigned ge = tiles<P, E>(l.nel) + record_blocks(ra.n, Shape<P, E>::NT);
     if constexpr (std::is_same<R, float>::value && E == 0) {
         if (l.bf16_static) {
-            if (l.vm == 6) return launch_ll<P, 0, float, 6, true>(l.ks, 0, ea, ra, st, ge);
-            if (l.vm == 5) return launch_ll<P, 0, float, 5, true>(l.ks, 0, ea, ra, st, ge);
-            return launch_ll<P, 0, float, 0, true>(l.ks, 0, ea, ra, st, ge);
+            if (l.vm == 6) return launch_ks<P, 0, float, 6, true>(l.ks, ea, ra, st, ge);
+            if (l.vm == 5) return launch_ks<P, 0, float, 5, true>(l.ks, ea, ra, st, ge);
+            return launch_ks<P, 0, float, 0, true>(l.ks, ea, ra, st, ge);
         }
     }
-    if (l.vm == 6) return launch_ll<P, E, R, 6, false>(l.ks, l.ll, ea, ra, st, ge);
-    if (l.vm == 5) return launch_ll<P, E, R, 5, false>(l.ks, l.ll, ea, ra, st, ge);
-    launch_ll<P, E, R, 0, false>(l.ks, l.ll, ea, ra, st, ge);
+    if (l.vm == 6) return launch_ks<P, E, R, 6, false>(l.ks, ea, ra, st, ge);
+    if (l.vm == 5) return launch_ks<P, E, R, 5, false>(l.ks, ea, ra, st, ge);
+    launch_ks<P, E, R, 0, false>(l.ks, ea, ra, st, ge);
 }
 
 template <int P, int E, typename R, int VM, int KS>
-void batch_ll(const ElemBatchLaunch &l, hipStream_t st)
+void batch(const ElemBatchLaunch &l, hipStream_t st)
 {
     constexpr int NT = Shape<P, E>::NT;
-    const ElemArgs<R> *args = (const ElemArgs<R> *)l.args;
-    const RecArgs<R> *recs = (const RecArgs<R> *)l.recs;
     const unsigned nwg = l.nwg + record_blocks(l.nrec, NT);
-    if constexpr (std::is_same<R, float>::value) {
-        if (l.ll == 1) {
-            hipLaunchKernelGGL((elem_kernel_batch<P, E, R, VM, KS, 1>), dim3(nwg), dim3(NT), 0, st, args, l.own, recs,
-                               l.rown, l.nrec);
-            return;
-        }
-        if (l.ll == 2) {
-            hipLaunchKernelGGL((elem_kernel_batch<P, E, R, VM, KS, 2>), dim3(nwg), dim3(NT), 0, st, args, l.own, recs,
-                               l.rown, l.nrec);
-            return;
-        }
-    }
-    hipLaunchKernelGGL((elem_kernel_batch<P, E, R, VM, KS, 0>), dim3(nwg), dim3(NT), 0, st, args, l.own, recs,
-                               l.rown, l.nrec);
+    hipLaunchKernelGGL((elem_kernel_batch<P, E, R, VM, KS>), dim3(nwg), dim3(NT), (spare_lds<P, E, R, VM, false, KS>()),
+                       st, (const ElemArgs<R> *)l.args, l.own, (const RecArgs<R> *)l.recs, l.rown, l.nrec);
 }
 
 template <int P, int E, typename R, int VM>
 void batch_ks(const ElemBatchLaunch &l, hipStream_t st)
 {
     if constexpr (std::is_same<R, float>::value) {
-        if (l.ks == 1) return batch_ll<P, E, R, VM, 1>(l, st);
-        if (l.ks == 2) return batch_ll<P, E, R, VM, 2>(l, st);
+        if (l.ks == 1) return batch<P, E, R, VM, 1>(l, st);
+        if (l.ks == 2) return batch<P, E, R, VM, 2>(l, st);
     }
-    batch_ll<P, E, R, VM, 0>(l, st);
+    batch<P, E, R, VM, 0>(l, st);
 }
 
 template <int P, int E, typename R>

@@ -41,6 +41,7 @@ namespace s3d {
 
 constexpr int MAXP1 = 8;       // p <= 7
 constexpr int NRDISS = 3;      // relaxation mechanisms
+constexpr int BLOCK_PAD = 16;  // bytes that 16-byte loads may read past the state and moduli blocks
 
 // Components of the element-major state block: stress (6), its compensation
 // (6 FP32 words for kahan_sigma 1, 3 packed BF16 pairs for 2) and the memory
@@ -51,6 +52,10 @@ constexpr int state_components(int kahan_sigma, int vm)
 {
     return 6 + (kahan_sigma == 1 ? 6 : kahan_sigma == 2 ? 3 : 0) + NRDISS * vm;
 }
+
+// Doubles of the coefficient table of order P1 - 1: Dx[i*P1+q] = 2 l_q'(xi_i) / dx,
+// Dy, Dz, dlw[i*P1+q] = l_i'(xi_q) w_q, then the GLL weights.
+constexpr int coef_words(int P1) { return 4 * P1 * P1 + P1; }
 
 // strain-rate / stress component order used everywhere: xx xy xz yy yz zz
 enum { XX = 0, XY, XZ, YY, YZ, ZZ };
@@ -126,9 +131,10 @@ struct ElemArgs {
     gptr<R> force;             // element force, k < p nodes then k = p layers (force_index)
     gptr<double> dgrad;        // [nel][6][NP] displacement gradient (xx xy xz yy yz zz) or null
     double dt;                 // time step (displacement gradient increment)
-    gptr<const ThTab<coef_t<R>>> tth;   // [nx*P1]
-    gptr<const RTab<coef_t<R>>> tr;     // [nz*P1]
-    gptr<const double> px, py, pz;  // 1-D taper profiles [n*P1]
+    // tables of the element kernel, in device memory: coefficients (the parts
+    // of coef_words), per theta element [4][P1] sin, 1/sin, cot, taper
+    // profile, per r element [4][P1] r, 1/r, r^2, taper profile, phi profile [ny*P1]
+    gptr<const double> coef, gx, gz, py;
     double alpha;              // taper slope
     int taper_on;
     gptr<const int> src_slot;  // [nel], -1 = none, or null
@@ -137,11 +143,6 @@ struct ElemArgs {
     gptr<const double> stf;    // [nchan][nt]
     coef_t<R> d1, d2, d3;      // (2/dx)J, (2/dy)J, -(2/dz)J
     R rate[NRDISS];            // dt/tau_p
-    coef_t<R> w[MAXP1];        // GLL weights
-    coef_t<R> Dx[MAXP1 * MAXP1];  // Dx[i*P1+q] = 2 l_q'(xi_i) / dx
-    coef_t<R> Dy[MAXP1 * MAXP1];
-    coef_t<R> Dz[MAXP1 * MAXP1];
-    coef_t<R> dlw[MAXP1 * MAXP1]; // dlw[i*P1+q] = l_i'(xi_q) w_q
 };
 
 template <typename R>

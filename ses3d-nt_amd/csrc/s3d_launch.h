@@ -21,16 +21,14 @@ struct ElemLaunch {
     long nel;          // elements
     int vm;            // memory words per relaxation mechanism: 0 (elastic), 6 or 5
     int ks;            // stress compensation: 0 off, 1 FP32 words, 2 BF16 words
-    int ll;            // kernel variant of the FP32 kernels: 0 planar LDS staging,
-                       // 1 node-interleaved staging, 2 planar with early state stores
-    int bf16_static;   // FP32 moduli and tau stored in BF16 (default tile, variant 0)
+    int bf16_static;   // FP32 moduli and tau stored in BF16 (default tile)
     int epb;           // elements per workgroup, 0 the default tile
 };
 
 // One batched element launch: a group's argument blocks for the current
 // phase (device memory) and its workgroup -> (member, member's workgroup) map.
 struct ElemBatchLaunch {
-    int vm, ks, ll, epb;   // as in ElemLaunch, shared by the group's members
+    int vm, ks, epb;       // as in ElemLaunch, shared by the group's members
     unsigned nwg;          // element workgroups of the launch
     const void *args;      // ElemArgs<R>[members]
     const int2 *own;       // [nwg]

@@ -6,7 +6,8 @@ receivers."""
 import numpy as np
 import pytest
 
-from helpers import random_model, rel_l2, small_grid
+import oracle
+from helpers import random_model, random_unique, rel_l2, small_grid, unique_to_local
 from ses3d_amd import api
 from test_gpu_parity import FIELDS, PARAMS, _pair, _random_state
 
@@ -88,6 +89,47 @@ def test_workgroup_orders_match_oracle(shape):
     for f in FIELDS:
         assert rel_l2(s.get(f), o.get(f)) < 1e-5, (shape, f)
         assert np.array_equal(s.get(f), plain.get(f)), (shape, f)
+
+
+@pytest.mark.parametrize("lpd,tile", [(2, 0), (2, 1), (3, 1), (4, 0), (4, 1), (5, 1), (6, 0), (7, 0)])
+@pytest.mark.parametrize("ks,words", [(0, 0), (1, 0), (2, 0), (0, 5), (1, 5), (2, 5), (0, 6), (1, 6)])
+def test_tile_loads_at_every_alignment(lpd, tile, ks, words):
+    """The FP32 element kernel loads a tile's contiguous words in 16-byte
+    vectors, whatever word the tile starts at: tiles of 1 to 9 elements of 27
+    to 512 nodes and 6 to 30 words per node start at every place modulo 4, and
+    the last of 7 elements ends inside a tile of 2, 4 or 9. One state block
+    for odd, two for even compensation modes."""
+    grid = small_grid(nx=7, ny=1, nz=1, lpd=lpd, taper_width=0)
+    rng = np.random.default_rng(10 * lpd + ks)
+    model = random_model(grid, rng, visco=words > 0)
+    o = oracle.Oracle(grid)
+    s = api.Simulation(grid, "fp32", kahan_sigma=ks, memory_vars=words, state_buffers=1 if ks == 1 else 2)
+    for k, arr in model.items():
+        o.set_model(PARAMS[k][0], arr)
+        s.set_model(PARAMS[k][1], arr)
+    o.init()
+    s.init()
+    s.set_tile(tile)
+    for f in (api.VX, api.VY, api.VZ):
+        v = unique_to_local(random_unique(grid, rng, 1e-3), grid)
+        o.set(f, v)
+        s.set(f, v)
+    shp = o.shape
+    for f in range(api.SXX, api.SZZ + 1):
+        x = 1e5 * rng.standard_normal(shp)
+        o.set(f, x)
+        s.set(f, x)
+    for m in range(3 if words else 0):
+        x = [1e-9 * rng.standard_normal(shp) for _ in range(6)]
+        x[5] = -(x[0] + x[3])               # deviatoric: both forms hold it
+        for c in range(6):
+            o.set(api.MXX + 6 * m + c, x[c])
+            if words == 6 or c < 5:
+                s.set(api.MXX + 6 * m + c, x[c])
+    o.step(3)
+    s.step(3)
+    for f in FIELDS:
+        assert rel_l2(s.get(f), o.get(f)) < 1e-5, f
 
 
 def test_run_without_sources_or_receivers():
