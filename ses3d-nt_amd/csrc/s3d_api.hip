@@ -782,20 +782,21 @@ struct CflRun {
 // and host threads copy between it and the caller's array, each with two
 // pinned buffers, so that the copies of some chunks (and the first touch of
 // the caller's pages) run while the host link carries others. Reading, one
-// thread per IO_PER_THREAD chunks: 442 MB into fresh pages (a velocity
-// component at 96x96x48, order 4) take 35 ms on one thread, 14.9 ms on 4,
-// 12.3 ms on 8; 32 MB 2.6 ms on one, 1.8 ms on 3; in 2 MB chunks the 442 MB
-// take 13.5 ms, in 1 MB chunks 15.8 ms, but a 4 MB field 0.7 ms in place of
-// 0.8 ms. (One hipMemcpy from a device buffer: 44 ms, and 254 ms for a stress
-// component whose compensation the host subtracted.) Writing, two threads
-// reach what the link takes, 9.2 ms for the 442 MB (hipMemcpy: 16.4 ms), and
-// more only get in the way of a caller whose own threads still spin. Buffers
-// are taken from a process-wide list for the duration of one call, at most
-// IO_KEPT sets per device stay on it, and the last simulation of a device
-// frees them.
+// thread per IO_READ bytes: 442 MB into fresh pages (a velocity component at
+// 96x96x48, order 4) take 35 ms on one thread, 14.9 ms on 4, 12.3 ms on 8; 32 MB
+// 2.6 ms on one, 1.8 ms on 3; in 2 MB chunks the 442 MB take 13.5 ms, in 1 MB
+// chunks 15.8 ms, but a 4 MB field 0.7 ms in place of 0.8 ms. (One hipMemcpy
+// from a device buffer: 44 ms, and 254 ms for a stress component whose
+// compensation the host subtracted.) Writing, one thread, and a second from
+// IO_WRITE bytes on: two reach what the link takes, 9.2 ms for the 442 MB
+// (hipMemcpy: 16.4 ms), one 15.8 ms, but a second thread that the caller's own,
+// still spinning, keep off the CPUs costs a 7 MB field 1.8 ms in place of
+// 0.35 ms. Buffers are taken from a process-wide list for the duration of one
+// call, at most IO_KEPT sets per device stay on it, and the last simulation of
+// a device frees them.
 constexpr int IO_THREADS = 8;
 constexpr size_t IO_BYTES = 4u << 20, IO_LEAST = 1u << 20;
-constexpr long IO_PER_THREAD = 4;
+constexpr long IO_READ = 16L << 20, IO_WRITE = 64L << 20;
 constexpr size_t IO_KEPT = 2;
 
 struct IoBuffers {
@@ -907,10 +908,11 @@ struct IoChunk {
 };
 
 // For every chunk `start(chunk, buffer, event)`, then `finish` of the same
-// arguments, on up to `most` (at most IO_THREADS) host threads; a thread starts a chunk in its
-// second buffer before it finishes the one in its first.
+// arguments, on one host thread and one more per `each` bytes of the fields,
+// at most `most` (at most IO_THREADS); a thread starts a chunk in its second
+// buffer before it finishes the one in its first.
 template <typename S, typename F>
-int io_chunks(s3d_ctx *c, int fields, int most, S start, F finish)
+int io_chunks(s3d_ctx *c, int fields, int most, long each, S start, F finish)
 {
     const IoPlan p = io_plan(c, fields);
     const long total = p.ce * p.cn;
@@ -938,7 +940,7 @@ int io_chunks(s3d_ctx *c, int fields, int most, S start, F finish)
             e = finish(k[at ^ 1], (double *)b->buf[2 * t + (at ^ 1)], b->ev[2 * t + (at ^ 1)]);
         if (e != hipSuccess) bad.store(e);
     };
-    const int want = (int)std::min<long>({(long)most, 1 + total / IO_PER_THREAD,
+    const int want = (int)std::min<long>({(long)most, total, 1 + (long)sizeof(double) * c->nn * fields / each,
                                           std::max(1L, (long)std::thread::hardware_concurrency() / 2)});
     std::vector<std::thread> crew;
     try {
@@ -972,7 +974,7 @@ template <typename Src>
 int io_get(s3d_ctx *c, const Src &src, double *out)
 {
     return io_chunks(
-        c, 1, IO_THREADS,
+        c, 1, IO_THREADS, IO_READ,
         [&](const IoChunk &k, double *chunk, hipEvent_t ev) {
             hipLaunchKernelGGL(export_field<Src>, k.grid(), dim3(256), 0, c->stream, src, k.e0, k.ne, k.n0, k.nn, chunk);
             const hipError_t e = hipGetLastError();
@@ -993,7 +995,7 @@ template <typename Dst>
 int io_set(s3d_ctx *c, const Dst &dst, const double *in)
 {
     return io_chunks(
-        c, 1, 2,
+        c, 1, 2, IO_WRITE,
         [&](const IoChunk &k, double *chunk, hipEvent_t ev) {
             hipError_t e = hipEventSynchronize(ev);   // the buffer's last chunk
             if (e != hipSuccess) return e;
@@ -1062,7 +1064,7 @@ struct GradRun {
         a.inc_dt = inc_dt;
         a.jac = c->jac;
         return io_chunks(
-            c, 3, 2,
+            c, 3, 2, IO_WRITE,
             [&](const IoChunk &k, double *chunk, hipEvent_t ev) {
                 hipError_t e = hipEventSynchronize(ev);
                 if (e != hipSuccess) return e;
