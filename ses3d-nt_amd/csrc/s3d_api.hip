@@ -176,7 +176,7 @@ struct s3d_ctx {
     int kv = 0;                // velocity compensation words: 0 none, 1 FP32, 2 BF16
     int dev = 0;
     hipStream_t stream = nullptr;
-    double *stage[7] = {};
+    double *stage[7] = {};     // model parameters until s3d_init, element-major [e][NP]
     bool q_finite = false, abc_nonzero = false;
     // geometry (host, FP64)
     double knots[MAXP1], weights[MAXP1], dl[MAXP1 * MAXP1];
@@ -875,28 +875,29 @@ hipError_t io_buffer(IoBuffers *b, int t)
     return hipSuccess;
 }
 
-// Chunks of `fields` fields of NP x nel values that share one buffer: whole
-// rows of elements where IO_N node rows of them fit, else pieces of rows.
+// Chunks of `fields` fields of NP x nel values (nel: elements of the caller's
+// arrays) that share one buffer: whole rows of elements where IO_N node rows of
+// them fit, else pieces of rows.
 struct IoPlan {
     long ne, ce;   // elements per chunk, chunks along the elements
     int nn, cn;    // nodes per chunk, chunks along the nodes
 };
 
-IoPlan io_plan(const s3d_ctx *c, int fields)
+IoPlan io_plan(long nel, int NP, int fields)
 {
-    const size_t all = sizeof(double) * c->nn * fields;
+    const size_t all = sizeof(double) * nel * NP * fields;
     const long words = (long)(std::min(IO_BYTES, std::max(IO_LEAST, all / 8)) / sizeof(double)) / fields;
     IoPlan p;
-    if (c->nel * std::min(c->NP, IO_N) <= words) {
-        p.ne = c->nel;
-        p.nn = (int)std::min<long>(c->NP, words / c->nel);
-        if (p.nn < c->NP) p.nn = p.nn / IO_N * IO_N;
+    if (nel * std::min(NP, IO_N) <= words) {
+        p.ne = nel;
+        p.nn = (int)std::min<long>(NP, words / nel);
+        if (p.nn < NP) p.nn = p.nn / IO_N * IO_N;
     } else {
-        p.nn = std::min(c->NP, IO_N);
+        p.nn = std::min(NP, IO_N);
         p.ne = words / p.nn / IO_E * IO_E;
     }
-    p.ce = (c->nel + p.ne - 1) / p.ne;
-    p.cn = (c->NP + p.nn - 1) / p.nn;
+    p.ce = (nel + p.ne - 1) / p.ne;
+    p.cn = (NP + p.nn - 1) / p.nn;
     return p;
 }
 
@@ -912,9 +913,9 @@ struct IoChunk {
 // at most `most` (at most IO_THREADS); a thread starts a chunk in its second
 // buffer before it finishes the one in its first.
 template <typename S, typename F>
-int io_chunks(s3d_ctx *c, int fields, int most, long each, S start, F finish)
+int io_chunks(s3d_ctx *c, long nel, int fields, int most, long each, S start, F finish)
 {
-    const IoPlan p = io_plan(c, fields);
+    const IoPlan p = io_plan(nel, c->NP, fields);
     const long total = p.ce * p.cn;
     IoBuffers *b = io_acquire(c->dev);
     std::atomic<long> next(0);
@@ -926,7 +927,7 @@ int io_chunks(s3d_ctx *c, int fields, int most, long each, S start, F finish)
         for (long q; e == hipSuccess && bad.load() == hipSuccess && (q = next.fetch_add(1)) < total; at ^= 1) {
             // consecutive chunks lie side by side in the caller's rows
             k[at].e0 = q % p.ce * p.ne;
-            k[at].ne = (int)std::min(p.ne, c->nel - k[at].e0);
+            k[at].ne = (int)std::min(p.ne, nel - k[at].e0);
             k[at].n0 = (int)(q / p.ce) * p.nn;
             k[at].nn = std::min(p.nn, c->NP - k[at].n0);
             e = io_buffer(b, 2 * t + at);
@@ -940,7 +941,7 @@ int io_chunks(s3d_ctx *c, int fields, int most, long each, S start, F finish)
             e = finish(k[at ^ 1], (double *)b->buf[2 * t + (at ^ 1)], b->ev[2 * t + (at ^ 1)]);
         if (e != hipSuccess) bad.store(e);
     };
-    const int want = (int)std::min<long>({(long)most, total, 1 + (long)sizeof(double) * c->nn * fields / each,
+    const int want = (int)std::min<long>({(long)most, total, 1 + (long)sizeof(double) * nel * c->NP * fields / each,
                                           std::max(1L, (long)std::thread::hardware_concurrency() / 2)});
     std::vector<std::thread> crew;
     try {
@@ -959,13 +960,13 @@ int io_chunks(s3d_ctx *c, int fields, int most, long each, S start, F finish)
 }
 
 // rows of a chunk between the pinned buffer and the caller's field
-void io_copy(const s3d_ctx *c, const IoChunk &k, double *field, double *chunk, bool out)
+void io_copy(long nel, const IoChunk &k, double *field, double *chunk, bool out)
 {
-    double *f = field + (size_t)k.n0 * c->nel + k.e0;
-    const long rows = k.ne == c->nel ? 1 : k.nn;
+    double *f = field + (size_t)k.n0 * nel + k.e0;
+    const long rows = k.ne == nel ? 1 : k.nn;
     const size_t words = (size_t)k.ne * k.nn / rows;
     for (long r = 0; r < rows; ++r) {
-        double *a = f + r * c->nel, *b = chunk + r * words;
+        double *a = f + r * nel, *b = chunk + r * words;
         std::memcpy(out ? a : b, out ? b : a, words * sizeof(double));
     }
 }
@@ -974,7 +975,7 @@ template <typename Src>
 int io_get(s3d_ctx *c, const Src &src, double *out)
 {
     return io_chunks(
-        c, 1, IO_THREADS, IO_READ,
+        c, c->nel, 1, IO_THREADS, IO_READ,
         [&](const IoChunk &k, double *chunk, hipEvent_t ev) {
             hipLaunchKernelGGL(export_field<Src>, k.grid(), dim3(256), 0, c->stream, src, k.e0, k.ne, k.n0, k.nn, chunk);
             const hipError_t e = hipGetLastError();
@@ -982,7 +983,7 @@ int io_get(s3d_ctx *c, const Src &src, double *out)
         },
         [&](const IoChunk &k, double *chunk, hipEvent_t ev) {
             const hipError_t e = hipEventSynchronize(ev);
-            if (e == hipSuccess) io_copy(c, k, out, chunk, true);
+            if (e == hipSuccess) io_copy(c->nel, k, out, chunk, true);
             return e;
         });
 }
@@ -991,15 +992,16 @@ int io_get(s3d_ctx *c, const Src &src, double *out)
 // use waits for it, and io_chunks for the last
 hipError_t io_no_finish(const IoChunk &, double *, hipEvent_t) { return hipSuccess; }
 
+// nel elements, the caller's and the destination's first ones the same
 template <typename Dst>
-int io_set(s3d_ctx *c, const Dst &dst, const double *in)
+int io_set(s3d_ctx *c, const Dst &dst, const double *in, long nel)
 {
     return io_chunks(
-        c, 1, 2, IO_WRITE,
+        c, nel, 1, 2, IO_WRITE,
         [&](const IoChunk &k, double *chunk, hipEvent_t ev) {
             hipError_t e = hipEventSynchronize(ev);   // the buffer's last chunk
             if (e != hipSuccess) return e;
-            io_copy(c, k, const_cast<double *>(in), chunk, false);
+            io_copy(nel, k, const_cast<double *>(in), chunk, false);
             hipLaunchKernelGGL(import_field<Dst>, k.grid(), dim3(256), 0, c->stream, dst, k.e0, k.ne, k.n0, k.nn, chunk);
             e = hipGetLastError();
             return e == hipSuccess ? hipEventRecord(ev, c->stream) : e;
@@ -1038,7 +1040,7 @@ struct UniqueSetRun {
         d.nx = c->g.nx;
         d.ny = c->g.ny;
         d.nz = c->g.nz;
-        return io_set(c, d, in);
+        return io_set(c, d, in, c->nel);
     }
 };
 
@@ -1064,12 +1066,12 @@ struct GradRun {
         a.inc_dt = inc_dt;
         a.jac = c->jac;
         return io_chunks(
-            c, 3, 2, IO_WRITE,
+            c, c->nel, 3, 2, IO_WRITE,
             [&](const IoChunk &k, double *chunk, hipEvent_t ev) {
                 hipError_t e = hipEventSynchronize(ev);
                 if (e != hipSuccess) return e;
                 for (int q = 0; q < 3; ++q)
-                    io_copy(c, k, const_cast<double *>(fw[q]), chunk + (size_t)q * k.ne * k.nn, false);
+                    io_copy(c->nel, k, const_cast<double *>(fw[q]), chunk + (size_t)q * k.ne * k.nn, false);
                 hipLaunchKernelGGL((grad_rho_kernel<P, R>), k.grid(), dim3(256), 0, c->stream, a, k.e0, k.ne, k.n0,
                                    k.nn, chunk);
                 e = hipGetLastError();
@@ -1756,24 +1758,25 @@ int s3d_set_model_slab(s3d_ctx *c, int param, int ez0, int nez, const double *da
     if (c->inited) return fail("model must be set before s3d_init");
     if (ez0 < 0 || nez < 1 || ez0 + nez > c->g.nz) return fail("slab outside the mesh");
     HIPCHK(hipSetDevice(c->dev));
+    const long layer = (long)c->g.nx * c->g.ny;
     if (!c->stage[param]) {
         if (dalloc(c, (void **)&c->stage[param], sizeof(double) * c->nn, false)) return 1;
         c->bytes -= sizeof(double) * (double)c->nn;   // staging is transient
-        if (param == S3D_Q) {
-            // default HUGE everywhere (src/model_paras.F90:76)
-            std::vector<double> h(c->nel, HUGE64);
-            for (int n = 0; n < c->NP; ++n)
-                HIPCHK(hipMemcpy(c->stage[param] + (size_t)n * c->nel, h.data(), sizeof(double) * c->nel,
-                                 hipMemcpyHostToDevice));
-        } else {
-            HIPCHK(hipMemset(c->stage[param], 0, sizeof(double) * c->nn));
+        if (nez < c->g.nz) {
+            // elements never set: Q = HUGE (src/model_paras.F90:76), else 0
+            hipLaunchKernelGGL(fill_kernel, dim3(nblocks(c->nn, 256)), dim3(256), 0, c->stream, c->stage[param],
+                               c->nn, param == S3D_Q ? HUGE64 : 0.0);
+            HIPCHK(hipGetLastError());
         }
     }
-    const size_t layer = (size_t)c->g.nx * c->g.ny;
-    const size_t width = layer * nez * sizeof(double);
-    HIPCHK(hipMemcpy2D(c->stage[param] + layer * ez0, sizeof(double) * c->nel, data, width, width,
-                       c->NP, hipMemcpyHostToDevice));
-    const size_t n = layer * nez * c->NP;
+    // the staged parameters are element-major, [e][NP]
+    BlockDst<double> d;
+    d.p = (decltype(d.p))(c->stage[param] + layer * ez0 * c->NP);
+    d.lo = nullptr;
+    d.nc = 1;
+    d.NP = c->NP;
+    if (io_set(c, d, data, layer * nez)) return 1;
+    const size_t n = (size_t)layer * nez * c->NP;
     if (param == S3D_Q) {
         for (size_t q = 0; q < n; ++q)
             if (data[q] != HUGE64) { c->q_finite = true; break; }
@@ -2277,14 +2280,14 @@ static int set_state(s3d_ctx *c, int field, const double *in)
             t.half = q % 2;
             t.nc = c->ns;
             t.NP = c->NP;
-            return io_set(c, t, in);
+            return io_set(c, t, in, c->nel);
         }
         d.p = (decltype(d.p))((R *)c->sig + NP * q);
         if (c->sig_lo) d.lo = (decltype(d.lo))((R *)c->sig_lo + NP * q);
     } else {
         d.p = (decltype(d.p))((R *)c->mem + NP * mem_word(c, field));
     }
-    return io_set(c, d, in);
+    return io_set(c, d, in, c->nel);
 }
 
 extern "C" {

@@ -504,7 +504,15 @@ __device__ inline S narrow(double x)
         return (S)x;
 }
 
-// Material from the FP64 staging arrays in reference layout: tau
+__global__ void __launch_bounds__(256) fill_kernel(double *p, long n, double x)
+{
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < n) p[t] = x;
+}
+
+// Material from the FP64 staging arrays (element-major, as all that follow:
+// the set-up kernels then read and write along the nodes; in the reference
+// layout every lane fetched a line of its own): tau
 // (= 6.0814 Q^-1.015, src/model_paras.F90:407), rho, dt*A, dt*B, dt*C and the
 // moduli times dt, elastic: lambda, mu; visco-elastic (dtau non-null):
 // kappa - 2 mu_tau / 3 = lambda - 2/3 tau mu and mu_tau = mu (1 + tau)
@@ -521,7 +529,7 @@ __global__ void material_kernel(const double *rhoinv, const double *lam, const d
     if (t >= nel * NP) return;
     long e = t / NP;
     int n = (int)(t - e * NP);
-    long s = (long)n * nel + e;
+    const long s = t;
     long tm = em_index(e, ncm, 0, NP, n);   // lam/mu/tau: element-major block of ncm
     const double l = lam ? lam[s] : 0.0, m = mu ? mu[s] : 0.0;
     if (dtau) {
@@ -564,7 +572,6 @@ __global__ void mass_kernel(const double *rhoinv, const double *sin_t, const dou
         mm64[t] = 0.0;
         return;
     }
-    const long nel = (long)nx * ny * nz;
     bool px[2] = {bx < nx, li == 0 && bx > 0};
     bool py[2] = {by < ny, lj == 0 && by > 0};
     bool pz[2] = {bz < nz, lk == 0 && bz > 0};
@@ -584,7 +591,7 @@ __global__ void mass_kernel(const double *rhoinv, const double *sin_t, const dou
                 int i = li + dx * P, j = lj + dy * P, k = lk + dz * P;
                 long e = ex + (long)nx * (ey + (long)ny * ez);
                 int n = i + P1 * (j + P1 * k);
-                double ri = rhoinv ? rhoinv[(long)n * nel + e] : 0.0;
+                double ri = rhoinv ? rhoinv[e * (P1 * P1 * P1) + n] : 0.0;
                 double rho = ri > 0.0 ? 1.0 / ri : 0.0;
                 double r = rad[ez * P1 + k];
                 double ww = w[i] * w[j] * w[k];
@@ -613,7 +620,7 @@ __global__ void cfl_kernel(const double *rhoinv, const double *lam, const double
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     double m[3] = {0, 0, 0};
     if (t < nel * NP) {
-        long n = t / nel, e = t - n * nel;
+        const long e = t / NP, n = t - e * NP;
         int i = (int)(n % P1), j = (int)((n / P1) % P1), k = (int)(n / (P1 * P1));
         int ex = (int)(e % nx), ey = (int)((e / nx) % ny), ez = (int)(e / ((long)nx * ny));
         double ri = rhoinv ? rhoinv[t] : 0.0;
