@@ -467,6 +467,7 @@ NodeArgs<R> node_args(s3d_ctx *c)
     a.px = (decltype(a.px))(c->dpx); a.py = (decltype(a.py))(c->dpy); a.pz = (decltype(a.pz))(c->dpz);
     a.alpha = c->g.taper_slope;
     a.taper_on = c->g.taper_width > 0;
+    a.rows = by_rows<P, R>(c->kv, c->nblk);
     a.it_dev = (decltype(a.it_dev))(c->d_it);
     return a;
 }
@@ -633,7 +634,7 @@ int launch_step(s3d_ctx *c, bool first, bool last)
     ev_end(c, 0);
     advance_state(c);   // the receivers read the stress this step wrote
     NodeArgs<R> na = node_args<P, R>(c);
-    const unsigned gn = nblocks(c->nuniq, 256);
+    const unsigned gn = nblocks(node_lanes<P, R>(c->kv, c->nblk), 256);
     ev_begin(c, 1);
     if (c->kv == 1)
         hipLaunchKernelGGL((node_kernel<P, R, 1>), dim3(gn), dim3(256), 0, c->stream, na);
@@ -1325,7 +1326,7 @@ int batch_build_group_e(BatchGroup &G)
             r.sig = (decltype(r.sig))((const R *)state_parts(c, h ? w1 : w0).sig);
         }
         es[q + 1] = es[q] + (int)nblocks(c->nel, S::EPB);
-        ns[q + 1] = ns[q] + (int)nblocks(c->nuniq, 256);
+        ns[q + 1] = ns[q] + (int)nblocks(node_lanes<P, R>(c->kv, c->nblk), 256);
         rs[q + 1] = rs[q] + c->nrec_dev;
     }
     G.ewg = es[n];

@@ -157,7 +157,7 @@ struct NodeArgs {
     gptr<const bf16> dt_inv_mm16;  // the same in BF16 when dt_inv_mm is null
     gptr<const double> px, py, pz;
     double alpha;
-    int taper_on;
+    int taper_on, rows;        // rows: one lane per row of P nodes (by_rows)
     gptr<int> it_dev;          // iterations completed, advanced by the first lane
 };
 

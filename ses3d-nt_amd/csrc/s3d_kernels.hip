@@ -10,7 +10,7 @@
 //                stages the effective stress in LDS and contracts the weak
 //                divergence (K8). Writes the element force, the tapered
 //                stress and the memory variables; all HBM traffic coalesced.
-//   node_kernel  one lane per unique node. Sums the (up to 8) element copies
+//   node_kernel  one lane per unique node or row of them (node_rows). Sums the (up to 8) element copies
 //                of the force in the reference's theta -> phi -> r order
 //                (K10, src/communicate_fields.F90:48-79; deterministic, no
 //                atomics), multiplies by 1/M (K9), integrates the velocity
@@ -32,6 +32,45 @@ namespace s3d {
 // ---------------------------------------------------------------------------
 // node kernel: assembly, 1/M, velocity integration, taper
 // ---------------------------------------------------------------------------
+// Which form of the kernel: true for one lane per row of P nodes (row_body),
+// false for one per node (node_body). Neither reaches the copy rate: the
+// force copies of one node lie in up to 8 elements, 3.4 loads per node and
+// component at order 2, 1.95 at order 4. A row needs P / 2 + 2.5 of them per
+// node less address work, but keeps 3 P sums, velocities and compensation
+// words in registers and its lanes read P words apart. Measured, lane per
+// node and lane per row, in us:
+//   order 2, 100x100x64, FP32 words    161  116    60x60x40, BF16  41.3 30.2
+//   order 2, 60x60x30, FP64           41.5 36.4    60x60x40, none  23.5 18.7
+//   order 3, 61x53x31, no words       42.4 37.5    FP32 words      58.1 62.0
+//   order 4, 48x48x24, FP64            110   98    96x96x48, FP32   418  516
+//   order 4, 64x60x28, no words       92.0 82.1    64x60x28, FP32   112  140
+//   order 5, 37x29x19, FP64           76.1 70.9    48x40x24, FP32   106  121
+//   order 6, 28x28x14, FP64           64.2 67.1    40x36x20, FP32   110  134
+// Rows of few workgroups only wait longer: order 4, FP64, 6x6x4 6.4 and
+// 8.6, 12x12x8 7.8 and 9.1, 20x20x14 (106 thousand rows) 15.5 and 15.5; order
+// 5, 16x16x10 10.4 and 11.5, 28x28x16 (358 thousand) 24.0 and 23.9; order 3,
+// 32x32x20 (206 thousand) 12.5 and 12.9; order 2, 42x42x24 (185 thousand) 13.3
+// and 11.5. So rows from NODE_ROWS on, two workgroups for each CU.
+constexpr long NODE_ROWS = 131072;
+template <int P, typename R, int KV>
+constexpr bool node_rows() { return P <= 2 || (KV == 0 && P <= 5); }
+
+template <int P, typename R>
+bool by_rows(int kv, long nblk)
+{
+    const bool rows = kv == 0   ? node_rows<P, R, 0>()
+                      : kv == 1 ? node_rows<P, R, 1>()
+                                : node_rows<P, R, 2>();
+    return rows && nblk * (P * P) >= NODE_ROWS;
+}
+
+// Lanes of the node kernel of a mesh of nblk blocks.
+template <int P, typename R>
+long node_lanes(int kv, long nblk)
+{
+    return nblk * (by_rows<P, R>(kv, nblk) ? P * P : P * P * P);
+}
+
 // KV: compensated velocity integration, 0 off, 1 FP32 compensation words,
 // 2 BF16 compensation words (the term carries the rounding error of the
 // sum, below half an FP32 unit of it, so 8 bits of it keep the sum within
@@ -138,11 +177,137 @@ __device__ __forceinline__ void node_body(const NodeArgs<R> &a, long tid)
     }
 }
 
+// The same for one lane per row of P unique nodes along theta: no lane loads
+// a dx = 1 copy for the first node of an element under a predicate that idles
+// the rest of its wave, and the index arithmetic is done once per row. The
+// lane holds the row's sums, so it only pays while these fit: see node_rows.
+template <int P, typename R, int KV>
+__device__ __forceinline__ void row_body(const NodeArgs<R> &a, long tid)
+{
+    constexpr int P1 = P + 1;
+    constexpr int NL = P1 * P1, NM = NL * P;   // force layout, see force_index
+    if (tid >= a.nblk * (P * P)) return;
+    if (tid == 0) a.it_dev[0] = a.it_dev[0] + 1;
+    const unsigned t = (unsigned)tid;
+    const unsigned b = t / (P * P);
+    const unsigned o = t - b * (P * P);
+    const unsigned lj = o % P, lk = o / P;
+    const unsigned nx = a.nx, ny = a.ny, nz = a.nz;
+    const unsigned nbx = nx + 1, nby = ny + 1;
+    const unsigned bq = b / nbx;
+    const unsigned bx = b - bq * nbx, bz = bq / nby, by = bq - bz * nby;
+    if ((by == ny && lj) || (bz == nz && lk)) return;
+
+    // Copies of node li of the row: element (bx-dx, by-dy, bz-dz) at local
+    // (li+dx*P, lj+dy*P, lk+dz*P); dx = 1 only for li = 0. dz = 0 lies in the
+    // k < p part of the force, dz = 1 (lk = 0, local k = p) in the k = p layers
+    // (force_index). Only present copies are loaded; absent ones are +0, and
+    // adding +0 is exact: the sum equals the reference's theta -> phi -> r
+    // sweep.
+    const bool px0 = bx < nx, px1 = bx > 0;
+    const bool py0 = by < ny, py1 = lj == 0 && by > 0;
+    const bool pz0 = bz < nz, pz1 = lk == 0 && bz > 0;
+    const long top = (long)a.nel * 3 * NM;   // start of the k = p layers
+    R x[4][3][P], w[4][3];                   // (dy, dz): the row's values, dx = 1's
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        const int dy = m & 1, dz = m >> 1;
+        const bool here = (dy ? py1 : py0) && (dz ? pz1 : pz0);
+        const unsigned e = bx + nx * ((by - dy) + ny * (bz - dz)), j2 = dy ? P : lj;
+        const long row = dz ? top + (long)e * (3 * NL) + P1 * j2 : (long)e * (3 * NM) + P1 * (j2 + P1 * lk);
+        constexpr int step[2] = {NM, NL};
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            w[m][c] = R(0);
+#pragma unroll
+            for (int i = 0; i < P; ++i) x[m][c][i] = R(0);
+        }
+        if (here && px0)
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+#pragma unroll
+                for (int i = 0; i < P; ++i) x[m][c][i] = a.force[row + c * step[dz] + i];
+        if (here && px1)   // element e - 1, the row's last node
+#pragma unroll
+            for (int c = 0; c < 3; ++c) w[m][c] = a.force[row - 3 * (dz ? NL : NM) + c * step[dz] + P];
+    }
+    const long u = (long)t * P;
+    const int n = px0 ? P : 1;   // nodes of the row
+    R im[P], vv[3][P], cc[3][P];
+    R *v[3] = {a.vx, a.vy, a.vz};
+    R *l[3] = {a.lx, a.ly, a.lz};
+    bf16 *h[3] = {a.hx, a.hy, a.hz};
+    // the whole row also of a padding block: its other entries exist
+#pragma unroll
+    for (int i = 0; i < P; ++i) im[i] = a.dt_inv_mm ? a.dt_inv_mm[u + i] : (R)(float)a.dt_inv_mm16[u + i];
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int i = 0; i < P; ++i) {
+            vv[c][i] = v[c][u + i];
+            if constexpr (KV == 1) cc[c][i] = l[c][u + i];
+            if constexpr (KV == 2) cc[c][i] = (R)(float)h[c][u + i];
+        }
+    R dmp[P];   // 1 - taper
+#pragma unroll
+    for (int i = 0; i < P; ++i) dmp[i] = R(0);
+    if (a.taper_on) {
+        const double py = a.py[by < ny ? by * P1 + lj : ny * P1 - 1], pz = a.pz[bz < nz ? bz * P1 + lk : nz * P1 - 1];
+#pragma unroll
+        for (int i = 0; i < P; ++i) {
+            const double px = a.px[px0 ? bx * P1 + i : nx * P1 - 1];
+            if (px + py + pz != 0.0) dmp[i] = (R)taper_damp(px, py, pz, a.alpha);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+#pragma unroll
+        for (int i = 0; i < P; ++i) {
+            R s[4];
+#pragma unroll
+            for (int m = 0; m < 4; ++m) s[m] = i == 0 ? x[m][c][0] + w[m][c] : x[m][c][i];
+            const R acc = (s[0] + s[1]) + (s[2] + s[3]);
+            if constexpr (KV != 0)
+                kahan_add(vv[c][i], cc[c][i], acc * im[i]);
+            else
+                vv[c][i] = vv[c][i] + acc * im[i];
+            vv[c][i] = vv[c][i] - vv[c][i] * dmp[i];
+            if constexpr (KV != 0) cc[c][i] = cc[c][i] - cc[c][i] * dmp[i];
+        }
+        if (n == P) {
+#pragma unroll
+            for (int i = 0; i < P; ++i) {
+                v[c][u + i] = vv[c][i];
+                if constexpr (KV == 1) l[c][u + i] = cc[c][i];
+                if constexpr (KV == 2) h[c][u + i] = (bf16)(float)cc[c][i];
+            }
+        } else {
+            v[c][u] = vv[c][0];
+            if constexpr (KV == 1) l[c][u] = cc[c][0];
+            if constexpr (KV == 2) h[c][u] = (bf16)(float)cc[c][0];
+        }
+    }
+}
+
+template <int P, typename R, int KV>
+__device__ __forceinline__ void assemble(const NodeArgs<R> &a, long tid)
+{
+    if constexpr (node_rows<P, R, KV>())
+        if (a.rows) return row_body<P, R, KV>(a, tid);
+    node_body<P, R, KV>(a, tid);
+}
+
+// Workgroups in the element kernel's order (chunk_block), so that they read
+// the force from the L2 that its XCD wrote it to, and walk HBM as one window:
+// in plain order order 6, 40x36x20 took 115 us (now 109), order 7, 36x30x18
+// 109 (103), order 3, 61x53x31 44.8 (41.9), order 4, 24x24x16 15.4 (14.0);
+// order 4, 96x96x48 416 (418).
 template <int P, typename R, int KV>
 __global__ void __launch_bounds__(256)
 node_kernel(const NodeArgs<R> a)
 {
-    node_body<P, R, KV>(a, (long)blockIdx.x * blockDim.x + threadIdx.x);
+    const long tid = (long)chunk_block(blockIdx.x, gridDim.x, 1) * blockDim.x + threadIdx.x;
+    assemble<P, R, KV>(a, tid);
 }
 
 template <int P, typename R, int KV>
@@ -150,7 +315,8 @@ __global__ void __launch_bounds__(256)
 node_kernel_batch(const NodeArgs<R> *__restrict__ args, const int2 *__restrict__ own)
 {
     const int2 o = own[blockIdx.x];
-    node_body<P, R, KV>(args[o.x], (long)o.y * blockDim.x + threadIdx.x);
+    const long tid = (long)o.y * blockDim.x + threadIdx.x;
+    assemble<P, R, KV>(args[o.x], tid);
 }
 
 // Strain-rate parts of the curl receiver channels (reference record_rot_v*,

@@ -132,6 +132,44 @@ def test_tile_loads_at_every_alignment(lpd, tile, ks, words):
         assert rel_l2(s.get(f), o.get(f)) < 1e-5, f
 
 
+@pytest.mark.parametrize("lpd,precision,kahan_v,shape", [
+    (2, "fp32", False, (127, 1, 127)), (2, "fp32", True, (31, 31, 31)), (2, "fp32", "bf16", (1, 127, 127)),
+    (2, "fp64", False, (127, 127, 1)), (2, "fp32", True, (126, 127, 1)), (3, "fp32", False, (85, 1, 85)),
+    (3, "fp64", False, (29, 28, 27)), (3, "fp32", True, (28, 27, 26)), (4, "fp64", False, (63, 63, 1)),
+    (4, "fp32", False, (1, 62, 63)), (5, "fp32", False, (16, 17, 17))])
+def test_assembly_by_rows_and_by_nodes(lpd, precision, kahan_v, shape):
+    """The assembly takes one lane per row of nodes from 131072 rows on (order
+    2, uncompensated up to order 5) and one per node elsewhere: the oracle's
+    results at that line, at the last mesh before it, past it and, by nodes,
+    in chunks of workgroups with a tail; on meshes one element thick along
+    each axis; and the same values from a member of a batch."""
+    nx, ny, nz = shape
+    grid = small_grid(nx=nx, ny=ny, nz=nz, lpd=lpd, taper_width=0 if 1 in shape else 1, dt=0.02)
+    rng = np.random.default_rng(300 + 10 * lpd + nx)
+    model = random_model(grid, rng)
+    o, s = _pair(grid, model, precision=precision, kahan_v=kahan_v)
+    member = api.Simulation(grid, precision, kahan_v=kahan_v)
+    other = small_grid(nx=3, ny=2, nz=2, lpd=lpd)
+    small = api.Simulation(other, precision, kahan_v=kahan_v)
+    for x, m in ((member, model), (small, random_model(other, rng))):
+        for k, arr in m.items():
+            x.set_model(PARAMS[k][1], arr)
+        x.init()
+    _random_state(o, s, grid, rng)
+    for f in FIELDS:
+        member.set(f, o.get(f))
+    o.step(2)
+    s.step(2)
+    b = api.Batch([small, member])
+    b.step(2)
+    b.synchronize()
+    for f in FIELDS:
+        got = s.get(f)
+        assert rel_l2(got, o.get(f)) < (1e-11 if precision == "fp64" else 1e-5), f
+        assert np.array_equal(member.get(f), got), f
+    b.close()
+
+
 def test_run_without_sources_or_receivers():
     grid = small_grid(nx=3, ny=2, nz=2, nt=20)
     rng = np.random.default_rng(5)
