@@ -148,9 +148,7 @@ def load_sims(case, modes, slab, remap=True, tune=None, state_buffers=0, memory_
             sim.set_tile(tune[0])
             sim.set_lds_layout(tune[1])
         sim.tile, sim.remap, sim.layout = sim.tuning()
-        sim.early = sim.store_order()
-        log("[bench] %s tuning: %d elements per workgroup, XCD order %d, LDS layout %d, "
-            "early stores %d" % (name, sim.tile, sim.remap, sim.layout, sim.early))
+        log("[bench] %s tuning: %d elements per workgroup, XCD order %d" % (name, sim.tile, sim.remap))
         nrec = 0
         for s_ in case.sources:
             loc = sim.locate(s_.lat, s_.lon, s_.depth)
@@ -407,18 +405,16 @@ def batch_bench(args):
 def multi_source_bench(args):
     """Many sources sharing one Earth model: one simulation per source on a
     single copy of the model (Simulation.shared), advanced by s3d_batch_step
-    with the members' workgroups source-innermost, against the same
-    simulations stepped round robin (whole mesh per source, no sharing of
-    the static-field reads). More sources than --per-batch run as successive
+    (one launch per kernel for all of them, member after member), against
+    the same simulations stepped round robin. More sources than --per-batch run as successive
     batches of --per-batch (the state of 32 sources at 128x128x48 exceeds the
     GPU's memory); the rates count every source over the summed times."""
     mode = args.mode
     kw = dict(MODES[mode])
     if kw.pop("bf16_static"):
         raise SystemExit("BF16 static fields are not supported in a batch")
-    # one state block per source unless asked otherwise: with source-innermost
-    # batches the second block does not pay (80.05 against 80.64 ms/step for
-    # 16 sources in batches of 8), and one block fits 16 sources per batch
+    # one state block per source unless asked otherwise: it fits 16 sources per
+    # batch instead of 8
     nbuf = args.state_buffers or 1
     kw["state_buffers"] = nbuf
     kw["memory_vars"] = args.memory_vars
@@ -595,11 +591,8 @@ def main():
     s_state = mode_sizes(mode)[0]
     roof = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK, "unit": "GB/s",
             "frac": achieved / HBM_PEAK, "traffic": None,
-            "kernel": "elem_kernel<%d,%s,visco>, %d elements per workgroup, %s LDS layout, %s "
-                      "workgroup order, state stored %s the divergence"
-                      % (g.lpd, rtype, tile, "node-interleaved" if sims[mode].layout else "planar",
-                         "XCD-aware" if sims[mode].remap else "plain",
-                         "before" if sims[mode].early else "after"),
+            "kernel": "elem_kernel<%d,%s,visco>, %d elements per workgroup, %s workgroup order"
+                      % (g.lpd, rtype, tile, "XCD-aware" if sims[mode].remap else "plain"),
             "algorithmic_bytes_per_launch": eb,
             "algorithmic_bytes_per_node": eb / N,
             # the element force the element kernel writes for the node kernel
