@@ -49,7 +49,7 @@ typedef struct s3d_options {
                               0 off, 1 FP32 compensation words,
                               2 BF16 compensation words                   */
     int device;            /* HIP device ordinal                          */
-    int xcd_remap;         /* 1: give each XCD contiguous runs of elements */
+    int xcd_remap;         /* 1: give each XCD runs of consecutive elements */
     int bf16_static;       /* FP32: store the moduli, tau and dt/M in BF16 */
     int state_buffers;     /* stress, compensation and memory variables:
                               2 (and 0, the default): two blocks, each step
@@ -166,7 +166,8 @@ int s3d_init(s3d_ctx *ctx);
 int s3d_cfl(s3d_ctx *ctx, double *courant);
 
 /* Autotuner: times the element kernel's tiles (elements per workgroup) and the
- * XCD-aware block order on this mesh and keeps the fastest; *tile gets the
+ * block order (plain, or XCD-aware in chunks or in ranges) on this mesh and
+ * keeps the fastest; *tile gets the
  * elements per workgroup chosen and *ms the element kernel time
  * (s3d_get_tuning gives the rest). Needs the state at rest (after s3d_init,
  * before s3d_set_field and s3d_step): the trial launches then leave every

@@ -173,6 +173,7 @@ struct s3d_ctx {
     int ns = 6;    // components of the state block
     long nel, nn, nblk, nuniq;
     bool fp32 = false, visco = false, aniso = false, inited = false;
+    bool ranges = false;       // XCD-aware order in ranges, not chunks (chunk_block)
     int kv = 0;                // velocity compensation words: 0 none, 1 FP32, 2 BF16
     int dev = 0;
     hipStream_t stream = nullptr;
@@ -403,7 +404,7 @@ ElemArgs<R> elem_args(s3d_ctx *c, int rd = -1, int wr = -1)
     std::memset(&a, 0, sizeof(a));
     const int P1 = P + 1;
     a.nx = c->g.nx; a.ny = c->g.ny; a.nz = c->g.nz; a.nel = (int)c->nel;
-    a.remap = c->o.xcd_remap;
+    a.remap = !c->o.xcd_remap ? ORDER_PLAIN : c->ranges ? ORDER_RANGES : ORDER_CHUNKS;
     a.it_dev = (decltype(a.it_dev))(c->d_it);
     a.nt = c->g.nt;
     a.kahan_sigma = c->o.kahan_sigma;
@@ -549,10 +550,11 @@ int autotune_p(s3d_ctx *c, int *tile_out, double *ms_out)
     HIPCHK(hipEventCreate(&e0));
     HIPCHK(hipEventCreate(&e1));
     double best = 1e300;
-    int best_tile = c->epb, best_remap = c->o.xcd_remap;
+    int best_tile = c->epb, best_order = ORDER_PLAIN;
     for (int tile : tile_candidates<P>(c->o.bf16_static))
-        for (int remap = 0; remap < 2; ++remap) {
-            c->o.xcd_remap = remap;
+        for (int order : {ORDER_PLAIN, ORDER_CHUNKS, ORDER_RANGES}) {
+            c->o.xcd_remap = order != ORDER_PLAIN;
+            c->ranges = order == ORDER_RANGES;
             ElemArgs<R> ea = elem_args<P, R>(c);
             RecArgs<R> none = rec_args<R>(c);
             none.n = 0;
@@ -567,13 +569,14 @@ int autotune_p(s3d_ctx *c, int *tile_out, double *ms_out)
             if (ms / 3.0 < best) {
                 best = ms / 3.0;
                 best_tile = tile;
-                best_remap = remap;
+                best_order = order;
             }
         }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     c->epb = best_tile;
-    c->o.xcd_remap = best_remap;
+    c->o.xcd_remap = best_order != ORDER_PLAIN;
+    c->ranges = best_order == ORDER_RANGES;
     c->lds_layout = 0;
     c->early_stores = false;
     drop_graph(c);
@@ -1646,6 +1649,7 @@ int s3d_create(const s3d_grid *grid, const s3d_options *opt, s3d_ctx **out)
     c->nn = c->nel * c->NP;
     c->nblk = (long)(grid->nx + 1) * (grid->ny + 1) * (grid->nz + 1);
     c->nuniq = c->nblk * c->PB;
+    c->ranges = !c->fp32 && c->nn >= RANGE_NODES_FP64;
     gll_tables(c->p, c->knots, c->weights, c->dl);
     io_live(c->dev, 1);
     *out = c;
@@ -1700,6 +1704,7 @@ int s3d_create_shared(s3d_ctx *base, s3d_ctx **out)
     // mesh, options, host geometry and element tile of the model's simulation
     c->g = m->g;
     c->o = m->o;
+    c->ranges = m->ranges;
     c->nbuf = m->nbuf;
     c->nm = m->nm;
     c->p = m->p; c->P1 = m->P1; c->NP = m->NP; c->PB = m->PB;

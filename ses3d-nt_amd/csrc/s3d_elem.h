@@ -25,7 +25,7 @@ struct Shape {
 };
 
 // Workgroup order of the element kernel: dispatch deals consecutive workgroups
-// to the 8 XCDs in turn; with `on`, XCD x runs the tiles of chunks x, x + 8,
+// to the 8 XCDs in turn; with ORDER_CHUNKS, XCD x runs the tiles of chunks x, x + 8,
 // x + 16, ... of XCD_CHUNK consecutive tiles each. Neighbours along theta
 // (shared velocity and force nodes) still meet in one L2, and all XCDs work
 // in one window of memory (8 chunks) that moves through the state block. With
@@ -40,15 +40,30 @@ struct Shape {
 // A launch of at most XCD_RESIDENT workgroups is in flight as a whole, there
 // is no moving window, and what its XCD wrote in the last step may still be in
 // that L2: ranges (12x12x8, order 4, FP64: 12.8 us, 13.2 us with chunks; at
-// 2048 workgroups 25.5 and 26.2 us, at 4608 60.0 and 55.2 us).
+// 2048 workgroups 25.5 and 26.2 us, at 4608 60.0 and 55.2 us). A count that 8
+// does not divide takes them too: 256 steps of 12x12x8, whose node kernel has
+// 381 workgroups, 4.21 ms in plain order, 3.78 ms in ranges.
+// On the largest meshes the ranges win again, most likely where a plane
+// exceeds what the L2s and the Infinity Cache keep until the next one reads
+// its velocity: FP64 from about 5e7 nodes on (chunks and ranges, ms: 96x96x48
+// 4.51 4.41, 128x128x48 8.21 7.85, 160x160x96 24.6 22.6, 192x192x96 34.6 32.3;
+// 48x48x24 0.53 0.55). In FP32 it goes by the mesh (192x192x96 17.0 16.2,
+// 192x192x32 5.81 5.67, 128x128x96 8.05 7.97, but 160x160x96 11.9 12.5,
+// 96x96x48 2.12 2.25, 96x96x192 8.02 8.95), so chunks unless s3d_autotune
+// finds ranges faster.
 constexpr int XCD_CHUNK = 16;
 constexpr int XCD_RESIDENT = 2048;
+constexpr long RANGE_NODES_FP64 = 50000000;
+enum { ORDER_PLAIN, ORDER_CHUNKS, ORDER_RANGES };
 
 __device__ inline int chunk_block(int b, int G, int on)
 {
     constexpr int group = 8 * XCD_CHUNK;
-    if (!on) return b;
-    if (G <= XCD_RESIDENT) return (G & 7) ? b : (b & 7) * (G >> 3) + (b >> 3);
+    if (on == ORDER_PLAIN) return b;
+    if (on == ORDER_RANGES || G <= XCD_RESIDENT) {
+        const int q = G >> 3;   // the last G mod 8 workgroups keep their place
+        return b < 8 * q ? (b & 7) * q + (b >> 3) : b;
+    }
     if (b >= G / group * group) return b;
     const int g = b / group, r = b - g * group;
     return g * group + (r & 7) * XCD_CHUNK + (r >> 3);

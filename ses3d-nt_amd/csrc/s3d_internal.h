@@ -106,7 +106,7 @@ struct Static16 {
 template <typename R>
 struct ElemArgs {
     int nx, ny, nz, nel;
-    int remap;                 // XCD-aware block order (chunk_block)
+    int remap;                 // workgroup order, ORDER_* (chunk_block)
     gptr<const int> it_dev;    // iterations completed so far (device counter);
                                // this launch computes iteration *it_dev + 1
     int nt;

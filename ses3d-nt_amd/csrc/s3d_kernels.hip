@@ -306,7 +306,7 @@ template <int P, typename R, int KV>
 __global__ void __launch_bounds__(256)
 node_kernel(const NodeArgs<R> a)
 {
-    const long tid = (long)chunk_block(blockIdx.x, gridDim.x, 1) * blockDim.x + threadIdx.x;
+    const long tid = (long)chunk_block(blockIdx.x, gridDim.x, ORDER_CHUNKS) * blockDim.x + threadIdx.x;
     assemble<P, R, KV>(a, tid);
 }
 
